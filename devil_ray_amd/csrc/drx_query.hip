@@ -146,7 +146,17 @@ __global__ void k_quantize_nodes (const float4 *__restrict__ inner, int n_inner,
 // wavefront takes the next chunk from the queue counter whenever its current chunk is used up, so its
 // lanes refill across chunks until the last chunk is gone.  Same candidate sequence and results as one
 // lane per point, whatever the chunk size and launch form.
-constexpr int kLocateChunk = 1024;   // entries per chunk unless tuned (drx_locate_autotune)
+
+// Launch of a streamed walk whose caller and drx_locate_autotune set neither form nor chunk.  A chunk is worked
+// through by one wavefront, 64 entries at a time, so a call of few points is as long as one chunk: 500 points on a
+// 16^3 order-2 mesh take 84 us in chunks of 64 and 252 us in one of 1,024; 262,144 points 158 / 589 us (order 3
+// on 48^3: 334 / 880 us).  More than 64 entries pay only where lane refill matters: points in Morton order or the
+// learned start (an MLP round needs full wavefronts), and every resident wavefront with several rounds of work;
+// there the persistent launch wins too (4 M Morton-ordered points, order 3 / order 4: 1.70 / 1.81 ms against 1.78 /
+// 1.97 ms chunked by 256 and 1.94 / 2.30 ms by 64; 1 M: 0.77 / 0.72 ms against 0.72 / 0.76 ms by 64; learned, 8 M
+// plain: 5.80 ms against 6.79 ms by 64).  Unordered points of the plain walk gain nothing from refill, and at that
+// size 1,024 is as good as 64 (4 M, order 3: 3.56 ms against 3.65 ms).
+constexpr int kLocateChunk = 64, kLocateChunkRefill = 128, kLocateChunkLarge = 1024, kLocateRefillRounds = 4;
 
 // Wave-uniform pool of unclaimed processing-order entries [claimed, end) for the streamed kernels; `more`:
 // further chunks may come from the queue.
@@ -819,17 +829,17 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
       if (chunk == 0) chunk = t.chunk;
     }
   }
-  if (launch == DRX_LAUNCH_AUTO) launch = DRX_LAUNCH_CHUNKED;
-  if (chunk == 0) chunk = kLocateChunk;
+  const int64_t resident = (int64_t)compute_units (dev) * 4 * locate_waves_per_simd (P, cfg.polish, learned ? 3 : walk);
+  // (a chunk of 64 is for small n only, so the grid's work-item count, 64 per chunk, stays in 32 bits)
+  const bool large = n > 64 * kLocateRefillRounds * resident, ordered = learned || (opts && opts->coherent_order);
+  if (launch == DRX_LAUNCH_AUTO) launch = large && ordered && chunk == 0 ? DRX_LAUNCH_PERSISTENT : DRX_LAUNCH_CHUNKED;
+  if (chunk == 0) chunk = !large ? kLocateChunk : launch == DRX_LAUNCH_PERSISTENT ? kLocateChunkRefill : kLocateChunkLarge;
   if (chunk < 64 || chunk > (1 << 20)) return fail (DRX_ERR_ARG, "drx_locate: chunk %d outside [64, 2^20]", chunk);
   const int64_t n_chunks = (n + chunk - 1) / chunk;
   if (n_chunks > (1ll << 31) - 1) return fail (DRX_ERR_ARG, "drx_locate: too many chunks");
   int64_t grid_s = n_chunks;
   if (launch == DRX_LAUNCH_PERSISTENT)
-  {
-    const int64_t resident = (int64_t)compute_units (dev) * 4 * locate_waves_per_simd (P, cfg.polish, learned ? 3 : walk);
     grid_s = n_chunks < resident ? n_chunks : resident;
-  }
   else
     queue = nullptr;
   const dim3 g (nblk (n, 256)), b (256);
@@ -990,7 +1000,7 @@ int drx_locate_autotune (const drx_mesh *mesh, const drx_bvh *bvh, const float *
     return fail (DRX_ERR_HIP, "drx_locate_autotune: hipEventCreate");
   }
   float best = INFINITY;
-  int best_launch = DRX_LAUNCH_CHUNKED, best_chunk = kLocateChunk;
+  int best_launch = DRX_LAUNCH_CHUNKED, best_chunk = kLocateChunkRefill;
   for (int c = 0; c < 5 && rc == DRX_OK; ++c)
     for (int l = 0; l < 2 && rc == DRX_OK; ++l)
     {

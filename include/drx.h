@@ -145,7 +145,7 @@ typedef struct drx_locate_opts
   int32_t launch;             /* drx_launch: how drx_locate's streamed walks (binary, 8-wide per lane,
                                  learned start) are launched, and whether drx_volume_integrate takes the
                                  sample-parallel kernel; the results are the same either way */
-  int32_t chunk;              /* points per wavefront chunk for those walks (0: tuned, else 1024) */
+  int32_t chunk;              /* points per wavefront chunk for those walks (0: tuned, else by the number of points) */
   int32_t *polished;          /* device, nullable: drx_locate writes 1 where the point's accepted solution took
                                  the FP64 correction (condition estimate > cond_threshold), else 0 */
   int32_t mlp_fallback;       /* DRX_INIT_MLP: the plain start that takes over (and decides acceptance) when
@@ -162,7 +162,8 @@ typedef struct drx_locate_opts
 
 enum drx_launch
 {
-  DRX_LAUNCH_AUTO = 0,        /* the form drx_locate_autotune picked for this device, order and walk, else chunked */
+  DRX_LAUNCH_AUTO = 0,        /* the form drx_locate_autotune picked for this device, order and walk, else by the
+                                 number of points */
   DRX_LAUNCH_CHUNKED = 1,     /* one wavefront per chunk of points */
   DRX_LAUNCH_PERSISTENT = 2,  /* about one wavefront per resident slot; wavefronts take chunks from a queue */
   DRX_LAUNCH_SAMPLES = 3      /* drx_volume_integrate: several wavefronts per 64 rays locate and shade
