@@ -14,15 +14,30 @@ namespace drx
 {
 
 // =============================================================================================
-// Split: one 64-lane wavefront per element, the 33 control nets of the element in LDS.
+// Split: the 33 sub-boxes of every element.
 // Semantics of construct_bvh (data_model/mesh_utils.cpp:557-670): 32 times pick the box of largest
 // volume (surface area when the volume is 0; ties -> lowest index), split its SubRef at 0.5 along the
 // longest reference axis (ties -> lowest axis, :482-506), de Casteljau-split the net (mother keeps the
 // lower half, the copy at index `count` keeps the upper half; elem_ops.hpp:1346-1406), re-hull both.
 // Then scale every box by 1.000001f about its centre (range.hpp:161-173).
+//
+// One workgroup per element.  A sub-box's net depends on its path from the element alone (the halves taken, along
+// axis depth % 3: every split halves the longest reference axis, lowest first), so the boxes of the first five
+// levels are split level by level, all boxes of a level in parallel, before it is known which of them the
+// largest-first rule splits; the rule then runs on the 62 measures in registers.  A box below the fifth level that
+// it picks (at least one: the 32nd split) is split on demand from its level-4 ancestor's net.  Nets and hulls are
+// the ones the rule's own order gives, by the same operations.
+//
+// The rule's order (32 dependent splits of one net each, an argmax and LDS round trips per split) left a
+// wavefront waiting on latency, and 33 nets of LDS per element few wavefronts per CU; only the 16 level-4 nets and
+// one scratch net are held now (level 5 needs hulls only).  262,144 elements of order 3: 5.15 -> 1.08 ms (450 MB of
+// output at copy rate: 0.1 ms); 110,592 of mixed orders 1-4: 5.37 -> 0.83 ms.  What is left is mostly the
+// per-element rule and its on-demand splits, one wavefront each.
 // =============================================================================================
 constexpr int kSplitBoxes = 33;
-constexpr int kSplitGlobalBlocks = 512;   // workgroups of the order-7/8 split, each with its nets in global memory
+constexpr int kSplitNets = 17;      // the level-4 nets and the scratch net of on-demand splits
+constexpr int kSplitScratch = 16;
+constexpr int kSplitExtras = 8;    // on-demand splits the ranked path holds
 
 __device__ __forceinline__ float box_measure (const float *b)   // b: xmin,xmax,ymin,ymax,zmin,zmax
 {
@@ -41,108 +56,302 @@ __device__ __forceinline__ float box_measure (const float *b)   // b: xmin,xmax,
   return v;
 }
 
-// de Casteljau halving of every line of a net along `axis` (order P, nets of NPE_ stride per component):
-// lane t handles (component t / lines, line t % lines), 64 lanes per pass.  Running min/max of both halves
-// per component go to a/b mn/mx.
-template <int P>
-__device__ __forceinline__ void split_lines (float *mom, float *dau, int NPE_, int axis, int lane, float &lo_a,
-                                             float &hi_a, float &lo_b, float &hi_b)
+// Order-P layout: lanes per (net, component) group, one line per lane and pass, and the component stride of a
+// net in LDS (a pad that staggers the groups' banks costs more occupancy than it saves: order 3, 4 floats: +9%).
+template <int P> struct SplitOrd
 {
-  // Row c of the wavefront (lanes 16c .. 16c+15) takes component c's lines, 16 at a time; row 3 idles.
-  // Each lane's hulls of its lines then reduce within its row.
-  constexpr int N1 = P + 1, LINES = N1 * N1;
-  const int stride = (axis == 0) ? 1 : ((axis == 1) ? N1 : N1 * N1);
-  const int c = lane >> 4;
-  if (c > 2) return;
-  for (int l = lane & 15; l < LINES; l += 16)
+  static constexpr int N1 = P + 1, LINES = N1 * N1, NPE = N1 * N1 * N1;
+  static constexpr int G = P <= 3 ? 16 : P == 4 ? 32 : 64;
+  static constexpr int CS = NPE;   // order 8: 17 nets just fit the LDS
+};
+
+// One line of a net: halves it along its axis (both halves in a[] and b[]).
+template <int P> __device__ __forceinline__ void split_line (const float *m, int stride, float a[P + 1], float b[P + 1])
+{
+#pragma unroll
+  for (int ii = 0; ii <= P; ++ii) a[ii] = b[ii] = m[ii * stride];
+#pragma unroll
+  for (int r = 1; r <= P; ++r)
   {
-    const int u = l % N1, v = l / N1;   // the two other indices, lowest axis first
-    const int base = (axis == 0) ? (N1 * u + LINES * v) : ((axis == 1) ? (u + LINES * v) : (u + N1 * v));
-    float *m = mom + c * NPE_ + base, *d = dau + c * NPE_ + base;
-    float a[N1], b[N1];
+    // mother: new[ii] = .5 old[ii-1] + .5 old[ii] for ii >= r (descending, so old[ii-1] is still old)
 #pragma unroll
-    for (int ii = 0; ii < N1; ++ii) a[ii] = b[ii] = m[ii * stride];
+    for (int ii = P; ii >= r; --ii) a[ii] = a[ii - 1] * (1.0f - 0.5f) + a[ii] * 0.5f;
+    // daughter: new[ii] = .5 old[ii] + .5 old[ii+1] for ii <= P - r (ascending)
 #pragma unroll
-    for (int r = 1; r <= P; ++r)
+    for (int ii = 0; ii <= P - r; ++ii) b[ii] = b[ii] * (1.0f - 0.5f) + b[ii + 1] * 0.5f;
+  }
+}
+
+// First dof and stride of line l along `axis` (the p+1 dofs along the axis, the other two indices fixed).
+template <int P> __device__ __forceinline__ int line_base (int axis, int l)
+{
+  constexpr int N1 = P + 1;
+  const int u = l % N1, v = l / N1;   // the two other indices, lowest axis first
+  return axis == 0 ? N1 * l : axis == 1 ? u + N1 * N1 * v : l;
+}
+template <int P> __device__ __forceinline__ constexpr int line_stride (int axis)
+{
+  return axis == 0 ? 1 : axis == 1 ? P + 1 : (P + 1) * (P + 1);
+}
+
+// Min / max of the lanes' hull keys over a group of G lanes; the group's last lane ends with the result.  The
+// lanes' hulls are never NaN (fminf / fmaxf from +-inf skip NaN values), so integer keys reduce them exactly.
+template <int G> __device__ __forceinline__ float group_min (float f)
+{
+  int32_t v = row_reduce_min (float_key (f));
+  if constexpr (G >= 32) v = min (v, dpp_move_i<0x142, 0xA> (v, v));
+  if constexpr (G >= 64) v = min (v, dpp_move_i<0x143, 0xC> (v, v));
+  return key_float (v);
+}
+template <int G> __device__ __forceinline__ float group_max (float f)
+{
+  int32_t v = row_reduce_max (float_key (f));
+  if constexpr (G >= 32) v = max (v, dpp_move_i<0x142, 0xA> (v, v));
+  if constexpr (G >= 64) v = max (v, dpp_move_i<0x143, 0xC> (v, v));
+  return key_float (v);
+}
+
+// Splits component net `src` along `axis` with the lanes of one group (gl = lane in the group): the lower half to
+// lo_dst, the upper to hi_dst (nullptr: not kept; lo_dst may be src), and the halves' hulls to lo_hull / hi_hull
+// (min, max; nullptr: no hulls).  Lines are disjoint and each is read and written by one lane.
+template <int P>
+__device__ __forceinline__ void split_component (const float *src, float *lo_dst, float *hi_dst, int axis, int gl,
+                                                 float *lo_hull, float *hi_hull)
+{
+  constexpr int G = SplitOrd<P>::G, LINES = SplitOrd<P>::LINES;
+  const int stride = line_stride<P> (axis);
+  float lo_a = INFINITY, hi_a = -INFINITY, lo_b = INFINITY, hi_b = -INFINITY;
+#pragma unroll
+  for (int l0 = 0; l0 < LINES; l0 += G)
+  {
+    const int l = l0 + gl;
+    if (l < LINES)
     {
-      // mother: new[ii] = .5 old[ii-1] + .5 old[ii] for ii >= r (descending, so old[ii-1] is still old)
+      const int base = line_base<P> (axis, l);
+      float a[P + 1], b[P + 1];
+      split_line<P> (src + base, stride, a, b);
 #pragma unroll
-      for (int ii = P; ii >= r; --ii) a[ii] = a[ii - 1] * (1.0f - 0.5f) + a[ii] * 0.5f;
-      // daughter: new[ii] = .5 old[ii] + .5 old[ii+1] for ii <= P - r (ascending)
-#pragma unroll
-      for (int ii = 0; ii <= P - r; ++ii) b[ii] = b[ii] * (1.0f - 0.5f) + b[ii + 1] * 0.5f;
+      for (int ii = 0; ii <= P; ++ii)
+      {
+        if (lo_dst) lo_dst[base + ii * stride] = a[ii];
+        if (hi_dst) hi_dst[base + ii * stride] = b[ii];
+        lo_a = fminf (lo_a, a[ii]);
+        hi_a = fmaxf (hi_a, a[ii]);
+        lo_b = fminf (lo_b, b[ii]);
+        hi_b = fmaxf (hi_b, b[ii]);
+      }
     }
-#pragma unroll
-    for (int ii = 0; ii < N1; ++ii)
+  }
+  if (lo_hull)
+  {
+    lo_a = group_min<G> (lo_a);
+    hi_a = group_max<G> (hi_a);
+    lo_b = group_min<G> (lo_b);
+    hi_b = group_max<G> (hi_b);
+    if (gl == G - 1)
     {
-      m[ii * stride] = a[ii];
-      d[ii * stride] = b[ii];
-      lo_a = fminf (lo_a, a[ii]);
-      hi_a = fmaxf (hi_a, a[ii]);
-      lo_b = fminf (lo_b, b[ii]);
-      hi_b = fmaxf (hi_b, b[ii]);
+      lo_hull[0] = lo_a;
+      lo_hull[1] = hi_a;
+      hi_hull[0] = lo_b;
+      hi_hull[1] = hi_b;
     }
   }
 }
 
-template <int PMAX>
-__global__ void __launch_bounds__ (64) k_split (const int32_t *__restrict__ ctrl_idx, const float *__restrict__ values,
-                                                 const int32_t *__restrict__ orders, const int64_t *__restrict__ offsets,
-                                                 int order, int n_el, float *__restrict__ out_aabbs,
-                                                 int32_t *__restrict__ out_prims, float *__restrict__ out_subrefs)
+// The speculative levels of one element: level D splits its 2^D boxes.  Box k of level D has its net in slot
+// k * (16 >> D) and heap index 2^D + k; its lower child stays in the slot, its upper child takes the slot
+// 16 >> (D + 1) above (level 4 keeps no nets).  hulls: 6 floats per heap index.
+template <int P, int D>
+__device__ __forceinline__ void split_level (float *nets, float *hulls, int group, int n_groups, int gl)
 {
-  constexpr int NPE = (PMAX + 1) * (PMAX + 1) * (PMAX + 1);
-  constexpr int DPL = (NPE + 63) / 64;   // dofs per lane
-  __shared__ float nets[kSplitBoxes * 3 * NPE];
-
-  const int e = blockIdx.x;
-  if (e >= n_el) return;
-  const int lane = threadIdx.x;
-  const int p = orders ? orders[e] : order;
-  const int npe = (p + 1) * (p + 1) * (p + 1);
-  const int64_t off = offsets ? offsets[e] : (int64_t)e * npe;
-
-  // net 0 <- element control points; box 0 = hull
-  float mn[3] = { INFINITY, INFINITY, INFINITY }, mx[3] = { -INFINITY, -INFINITY, -INFINITY };
-#pragma unroll
-  for (int k = 0; k < DPL; ++k)
+  constexpr int CS = SplitOrd<P>::CS, AXIS = D % 3, STEP = 16 >> D;
+  for (int t = group; t < (3 << D); t += n_groups)
   {
-    const int d = lane + 64 * k;
-    if (d < npe)
-    {
-      const int64_t g = (int64_t)ctrl_idx[off + d] * 3;
+    const int k = t / 3, c = t - 3 * k;
+    float *net = nets + (k * STEP * 3 + c) * CS;
+    float *h = hulls + 6 * (2 * ((1 << D) + k)) + 2 * c;
+    if constexpr (D < 4)
+      split_component<P> (net, net, net + (STEP / 2) * 3 * CS, AXIS, gl, h, h + 6);
+    else
+      split_component<P> (net, nullptr, nullptr, AXIS, gl, h, h + 6);
+  }
+}
+
+__device__ __forceinline__ void split_wave_sync ()
+{
+  __builtin_amdgcn_fence (__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier ();
+  __builtin_amdgcn_fence (__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// On-demand split (one wavefront) of the box at `depth` >= 5 with path `path` (the halves taken, first split in
+// the highest of the depth bits): its net is halved out of its level-4 ancestor's into the scratch net, then the
+// hulls of its two halves go to hull_out[0..5] and [6..11].
+template <int P>
+__device__ __forceinline__ void split_deep (float *nets, float *hull_out, uint32_t path, int depth, int lane)
+{
+  constexpr int G = SplitOrd<P>::G, NG = 64 / G, CS = SplitOrd<P>::CS;
+  const int group = lane / G, gl = lane % G;
+  float *scratch = nets + kSplitScratch * 3 * CS;
+  const float *src = nets + (path >> (depth - 4)) * 3 * CS;
+  for (int d = 4; d < depth; ++d)
+  {
+    const bool upper = (path >> (depth - 1 - d)) & 1u;
+    for (int c = group; c < 3; c += NG)
+      split_component<P> (src + c * CS, upper ? nullptr : scratch + c * CS, upper ? scratch + c * CS : nullptr, d % 3, gl,
+                          nullptr, nullptr);
+    split_wave_sync ();
+    src = scratch;
+  }
+  for (int c = group; c < 3; c += NG)
+    split_component<P> (src + c * CS, nullptr, nullptr, depth % 3, gl, hull_out + 2 * c, hull_out + 6 + 2 * c);
+  split_wave_sync ();
+}
+
+// Writes box k of the output: the hull scaled by 1.000001f about its centre, and the SubRef from the path (every
+// split keeps one half along axis d % 3).
+__device__ __forceinline__ void split_emit (int64_t k, const float *hull, uint32_t path, int depth,
+                                            float *__restrict__ out_aabbs, float *__restrict__ out_subrefs)
+{
+  float ref[6] = { 0.f, 0.f, 0.f, 1.f, 1.f, 1.f };
+  for (int d = 0; d < depth; ++d)
+  {
+    const bool upper = (path >> (depth - 1 - d)) & 1u;
+    const int axis = d % 3;
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
+    for (int q = 0; q < 3; ++q)
+      if (q == axis)
       {
-        const float v = values[g + c];
-        nets[c * NPE + d] = v;
-        mn[c] = fminf (mn[c], v);
-        mx[c] = fmaxf (mx[c], v);
+        const float split_pt = ref[q] * (1.0f - 0.5f) + ref[3 + q] * 0.5f;
+        ref[q] = upper ? split_pt : ref[q];
+        ref[3 + q] = upper ? ref[3 + q] : split_pt;
       }
-    }
   }
-  // Per-box state lives in registers: lane b (< 33) holds box b's hull, SubRef and measure.
-  float my_box[6], my_ref[6], my_meas = -INFINITY;
+  const float s = (float)1.000001;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
   {
-    float b0[6];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
+    float lo = hull[2 * d], hi = hull[2 * d + 1];
+    if (!(lo > hi))
     {
-      b0[2 * c] = wave_reduce_min (mn[c]);
-      b0[2 * c + 1] = wave_reduce_max (mx[c]);
+      const float c = 0.5f * (lo + hi);
+      const float delta = s * 0.5f * (hi - lo);
+      const float v0 = c - delta, v1 = c + delta;
+      lo = fminf (lo, v0);
+      hi = fmaxf (hi, v0);
+      lo = fminf (lo, v1);
+      hi = fmaxf (hi, v1);
     }
-#pragma unroll
-    for (int q = 0; q < 6; ++q) my_box[q] = b0[q];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      my_ref[d] = 0.f;
-      my_ref[3 + d] = 1.f;
-    }
-    if (lane == 0) my_meas = box_measure (b0);
+    out_aabbs[6 * k + 2 * d] = lo;
+    out_aabbs[6 * k + 2 * d + 1] = hi;
+    out_subrefs[6 * k + d] = ref[d];
+    out_subrefs[6 * k + 3 + d] = ref[3 + d];
   }
-  __syncthreads ();
+}
 
+// The largest-first rule by ranks (one wavefront).  Where every box's measure is below its parent's and no two
+// measures tie, the rule splits the 32 boxes of largest measure, in order of measure, so a box's rank among the 63
+// is its place in that order: 63 broadcasts and compares instead of 32 dependent argmax reductions (262,144
+// elements of order 3: 1.59 -> 1.08 ms).
+// Box indices follow from the ranks: a lower child keeps its parent's index, an upper child takes the parent's
+// place + 1.  Returns false, with nothing written, where that does not hold (ties, NaN measures, a
+// box as large as its parent, a sixth-level box that would be split too, too many on-demand splits).
+template <int P>
+__device__ __forceinline__ bool split_ranked (float *nets, float *hulls, float *extra, float node_meas, int lane, int64_t k0,
+                                              float *__restrict__ out_aabbs, float *__restrict__ out_subrefs)
+{
+  const int32_t key = lane <= 1 ? INT32_MAX : float_key (node_meas);
+  if (__ballot (lane > 1 && !(node_meas == node_meas)) != 0) return false;
+  int rank = 0;
+#pragma unroll
+  for (int h = 1; h < 64; ++h) rank += (__builtin_amdgcn_readlane (key, h) > key) ? 1 : 0;
+  const bool split = lane >= 1 && rank < kSplitBoxes - 1;
+  const uint64_t split_mask = __ballot (split);
+  if (__popcll (split_mask) != kSplitBoxes - 1) return false;
+  // each place 0..31 taken once (a tie leaves the next place free), each split box after its parent
+  int32_t places = split ? (int32_t)(1u << rank) : 0;
+  places |= dpp_perm_i<0xB1> (places);
+  places |= dpp_perm_i<0x4E> (places);
+  places |= dpp_perm_i<0x141> (places);
+  places |= dpp_perm_i<0x140> (places);
+  places |= dpp_move_i<0x142, 0xA> (0, places);
+  places |= dpp_move_i<0x143, 0xC> (0, places);
+  if (__builtin_amdgcn_readlane (places, 63) != -1) return false;
+  const int parent_rank = __shfl (rank, lane >> 1, 64);
+  if (__ballot (split && lane > 1 && parent_rank >= rank) != 0) return false;
+  // box index: up to the first ancestor-or-self that is an upper child
+  int index = 0;
+  {
+    int h = lane;
+    bool open = lane > 1;
+#pragma unroll
+    for (int d = 0; d < 5; ++d)
+    {
+      const int pr = __shfl (rank, h >> 1, 64);
+      if (open && (h & 1))
+      {
+        index = pr + 1;
+        open = false;
+      }
+      h >>= 1;
+      if (h <= 1) open = false;
+    }
+  }
+  // on-demand splits of fifth-level boxes: their children must stay below the smallest box that is split
+  const uint64_t deep = split_mask >> 32;
+  const int n_deep = __popcll (deep);
+  if (n_deep > kSplitExtras) return false;
+  const int32_t least = __builtin_amdgcn_readlane (key, __ffsll ((unsigned long long)__ballot (split && rank == kSplitBoxes - 2)) - 1);
+  uint64_t todo = deep;
+  for (int x = 0; x < n_deep; ++x)
+  {
+    const int q = __ffsll ((unsigned long long)todo) - 1;
+    todo &= todo - 1;
+    split_deep<P> (nets, extra + 12 * x, (uint32_t)q, 5, lane);
+  }
+  {
+    float b[6];
+    bool big = false;
+    if (lane < 2 * n_deep)
+    {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) b[q] = extra[6 * lane + q];
+      const float m = box_measure (b);
+      big = !(m == m) || float_key (m) >= least;
+    }
+    if (__ballot (big) != 0) return false;
+  }
+  const bool parent_split = lane > 1 && ((split_mask >> (lane >> 1)) & 1ull) != 0;
+  if (parent_split && !split)
+  {
+    const int depth = 31 - __clz (lane);
+    split_emit (k0 + index, hulls + 6 * lane, (uint32_t)(lane - (1 << depth)), depth, out_aabbs, out_subrefs);
+  }
+  // the children of the boxes split on demand: lanes 2x, 2x + 1
+  {
+    uint64_t m = deep;
+    for (int x = 0; x < (lane >> 1); ++x) m &= m - 1;
+    const int h = lane < 2 * n_deep ? 32 + __ffsll ((unsigned long long)m) - 1 : 1;
+    const int hi = __shfl (index, h, 64), hr = __shfl (rank, h, 64);
+    if (lane < 2 * n_deep)
+      split_emit (k0 + ((lane & 1) ? hr + 1 : hi), extra + 6 * lane, (uint32_t)(2 * (h - 32) + (lane & 1)), 6, out_aabbs,
+                  out_subrefs);
+  }
+  return true;
+}
+
+// The largest-first rule as dray runs it (one wavefront).
+template <int P>
+__device__ __forceinline__ void split_sequential (float *nets, float *hulls, float node_meas, int lane, int64_t k0,
+                                                  float *__restrict__ out_aabbs, float *__restrict__ out_subrefs)
+{
+  // lane b (< 33): box b's path, depth and measure; the hull of a box from an on-demand split, else in `hulls`
+  uint32_t my_path = 0;
+  int my_depth = 0;
+  float my_meas = 0.f, my_box[6];   // box 0 is the element, split first whatever its measure
+#pragma unroll
+  for (int q = 0; q < 6; ++q) my_box[q] = 0.f;
+  bool own_box = false;
   for (int count = 1; count <= kSplitBoxes - 1; ++count)
   {
     // pick the box: dray's scan keeps the first strictly larger measure (ties -> lowest index; a NaN
@@ -160,328 +369,115 @@ __global__ void __launch_bounds__ (64) k_split (const int32_t *__restrict__ ctrl
         max_id = __ffsll ((unsigned long long)hit) - 1;
       }
     }
-    float sr[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) sr[q] = __int_as_float (__builtin_amdgcn_readlane (__float_as_int (my_ref[q]), max_id));
-    int axis = 0;
-    float maxlen = sr[3] - sr[0];
-    for (int d = 1; d < 3; ++d)
+    const uint32_t path = (uint32_t)__builtin_amdgcn_readlane ((int)my_path, max_id);
+    const int depth = __builtin_amdgcn_readlane (my_depth, max_id);
+    const bool low = lane == max_id, high = lane == count;
+    if (low || high)
     {
-      const float len = sr[3 + d] - sr[d];
-      if (len > maxlen)
-      {
-        axis = d;
-        maxlen = len;
-      }
+      my_path = 2 * path + (high ? 1u : 0u);
+      my_depth = depth + 1;
     }
-    const float split_pt = sr[axis] * (1.0f - 0.5f) + sr[3 + axis] * 0.5f;
-    if (lane == count)   // complement: lo[axis] = split
+    if (depth < 5)
     {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_ref[q] = (q == axis) ? split_pt : sr[q];
+      const int h = 2 * ((1 << depth) + (int)path);
+      const float ma = __int_as_float (__builtin_amdgcn_readlane (__float_as_int (node_meas), h));
+      const float mb = __int_as_float (__builtin_amdgcn_readlane (__float_as_int (node_meas), h + 1));
+      my_meas = low ? ma : high ? mb : my_meas;
     }
-    if (lane == max_id)   // in place: hi[axis] = split
-    {
-#pragma unroll
-      for (int d = 0; d < 3; ++d)
-        if (d == axis) my_ref[3 + d] = split_pt;
-    }
-    // split the mother's net along `axis`, one (line, component) per lane (component c in row c): a line is the p+1 dofs along
-    // the axis with the other two indices fixed; each lane reads its line, runs the de Casteljau rounds in
-    // registers (mother keeps [lo, mid], daughter [mid, hi]; the same operations in the same order as
-    // split_inplace, elem_ops.hpp:1346-1406) and writes both halves.  Lines are disjoint, so no lane
-    // reads what another lane writes in this count.
-    float *mom = nets + max_id * 3 * NPE;
-    float *dau = nets + count * 3 * NPE;
-    float lo_a = INFINITY, hi_a = -INFINITY, lo_b = INFINITY, hi_b = -INFINITY;
-    if constexpr (PMAX == 0)
-      ;
-    else if (p == PMAX)
-      split_lines<PMAX> (mom, dau, NPE, axis, lane, lo_a, hi_a, lo_b, hi_b);
     else
-      switch (p)   // mixed-order meshes
+    {
+      split_deep<P> (nets, hulls, path, depth, lane);   // heap indices 0 and 1 are free
+      if (low || high)
       {
-      case 1: split_lines<1> (mom, dau, NPE, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      case 2: split_lines<(PMAX >= 2 ? 2 : 1)> (mom, dau, NPE, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      case 3: split_lines<(PMAX >= 3 ? 3 : 1)> (mom, dau, NPE, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      default: split_lines<(PMAX >= 4 ? 4 : 1)> (mom, dau, NPE, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) my_box[q] = hulls[(high ? 6 : 0) + q];
+        my_meas = box_measure (my_box);
+        own_box = true;
       }
-    // the lanes' hulls are never NaN (fminf / fmaxf from +-inf skip NaN values), so their integer keys
-    // reduce exactly like the floats
-    const int32_t klo_a = row_reduce_min (float_key (lo_a)), khi_a = row_reduce_max (float_key (hi_a));
-    const int32_t klo_b = row_reduce_min (float_key (lo_b)), khi_b = row_reduce_max (float_key (hi_b));
-    float ba[6], bb[6];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-    {
-      ba[2 * c] = key_float (__builtin_amdgcn_readlane (klo_a, 16 * c));
-      ba[2 * c + 1] = key_float (__builtin_amdgcn_readlane (khi_a, 16 * c));
-      bb[2 * c] = key_float (__builtin_amdgcn_readlane (klo_b, 16 * c));
-      bb[2 * c + 1] = key_float (__builtin_amdgcn_readlane (khi_b, 16 * c));
+      split_wave_sync ();
     }
-    if (lane == max_id)
-    {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_box[q] = ba[q];
-      my_meas = box_measure (ba);
-    }
-    if (lane == count)
-    {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_box[q] = bb[q];
-      my_meas = box_measure (bb);
-    }
-    __syncthreads ();
   }
 
   if (lane < kSplitBoxes)
   {
-    float b[6];
-    for (int q = 0; q < 6; ++q) b[q] = my_box[q];
-    const float s = (float)1.000001;
+    if (!own_box)
+    {
+      const int h = (1 << my_depth) + (int)my_path;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      float lo = b[2 * d], hi = b[2 * d + 1];
-      if (!(lo > hi))
-      {
-        const float c = 0.5f * (lo + hi);
-        const float delta = s * 0.5f * (hi - lo);
-        const float v0 = c - delta, v1 = c + delta;
-        lo = fminf (lo, v0);
-        hi = fmaxf (hi, v0);
-        lo = fminf (lo, v1);
-        hi = fmaxf (hi, v1);
-      }
-      b[2 * d] = lo;
-      b[2 * d + 1] = hi;
+      for (int q = 0; q < 6; ++q) my_box[q] = hulls[6 * h + q];
     }
-    const int64_t k = (int64_t)e * kSplitBoxes + lane;
-    for (int q = 0; q < 6; ++q)
-    {
-      out_aabbs[6 * k + q] = b[q];
-      out_subrefs[6 * k + q] = my_ref[q];
-    }
-    out_prims[k] = e;
+    split_emit (k0 + lane, my_box, my_path, my_depth, out_aabbs, out_subrefs);
   }
 }
 
-// The same split with one wavefront per component (a 192-thread workgroup per element), for orders >= 4, where
-// the 33 nets take 49.5 KB of LDS (order 4) and allow only 3 elements per CU: each wavefront splits only its own
-// component's lines (one line per lane, one pass), reduces that component's two hulls over the wave, and the
-// three wavefronts exchange the six values through LDS once per split.  A wavefront reads and writes only its
-// own component's part of the nets, so the exchange is the only synchronisation.  Every wavefront keeps the
-// same box state (hulls, SubRefs, measures) and takes the same decisions; wavefront 0 writes the result.
-template <int P>
-__device__ __forceinline__ void split_lines_comp (float *mom, float *dau, int axis, int lane, float &lo_a,
-                                                  float &hi_a, float &lo_b, float &hi_b)
+template <int P, int WAVES>
+__device__ __forceinline__ void split_element (const int32_t *__restrict__ ctrl_idx, const float *__restrict__ values,
+                                               int64_t off, int e, float *nets, float *hulls, float *extra,
+                                               float *__restrict__ out_aabbs, int32_t *__restrict__ out_prims,
+                                               float *__restrict__ out_subrefs)
 {
-  constexpr int N1 = P + 1, LINES = N1 * N1;
-  const int stride = (axis == 0) ? 1 : ((axis == 1) ? N1 : N1 * N1);
-  for (int l = lane; l < LINES; l += 64)   // one pass up to order 7, two at order 8
+  constexpr int G = SplitOrd<P>::G, CS = SplitOrd<P>::CS, NPE = SplitOrd<P>::NPE;
+  const int lane = threadIdx.x & 63;
+  for (int d = threadIdx.x; d < NPE; d += 64 * WAVES)
   {
-    const int u = l % N1, v = l / N1;
-    const int base = (axis == 0) ? (N1 * u + LINES * v) : ((axis == 1) ? (u + LINES * v) : (u + N1 * v));
-    float *m = mom + base, *d = dau + base;
-    float a[N1], b[N1];
+    const int64_t g = (int64_t)ctrl_idx[off + d] * 3;
 #pragma unroll
-    for (int ii = 0; ii < N1; ++ii) a[ii] = b[ii] = m[ii * stride];
-#pragma unroll
-    for (int r = 1; r <= P; ++r)
-    {
-#pragma unroll
-      for (int ii = P; ii >= r; --ii) a[ii] = a[ii - 1] * (1.0f - 0.5f) + a[ii] * 0.5f;
-#pragma unroll
-      for (int ii = 0; ii <= P - r; ++ii) b[ii] = b[ii] * (1.0f - 0.5f) + b[ii + 1] * 0.5f;
-    }
-#pragma unroll
-    for (int ii = 0; ii < N1; ++ii)
-    {
-      m[ii * stride] = a[ii];
-      d[ii * stride] = b[ii];
-      lo_a = fminf (lo_a, a[ii]);
-      hi_a = fmaxf (hi_a, a[ii]);
-      lo_b = fminf (lo_b, b[ii]);
-      hi_b = fmaxf (hi_b, b[ii]);
-    }
-  }
-}
-
-// GNETS (orders 7 and 8, whose nets exceed the LDS): the nets live in a global scratch area, one per
-// workgroup, and each workgroup takes elements blockIdx.x, blockIdx.x + gridDim.x, ...
-template <int PMAX, bool GNETS>
-__global__ void __launch_bounds__ (192) k_split_cw (const int32_t *__restrict__ ctrl_idx, const float *__restrict__ values,
-                                                    const int32_t *__restrict__ orders, const int64_t *__restrict__ offsets,
-                                                    int order, int n_el, float *__restrict__ out_aabbs,
-                                                    int32_t *__restrict__ out_prims, float *__restrict__ out_subrefs,
-                                                    float *__restrict__ gnets)
-{
-  constexpr int NPE = (PMAX + 1) * (PMAX + 1) * (PMAX + 1);
-  __shared__ float lnets[GNETS ? 1 : kSplitBoxes * 3 * NPE];   // box b, component c at (b * 3 + c) * NPE
-  __shared__ float xch[2][3][4];                                // per split parity: each component's hull pair
-  float *nets = GNETS ? gnets + (size_t)blockIdx.x * kSplitBoxes * 3 * NPE : lnets;
-  const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int e = blockIdx.x; e < n_el; e += gridDim.x)
-  {
-  const int p = orders ? orders[e] : order;
-  const int npe = (p + 1) * (p + 1) * (p + 1);
-  const int64_t off = offsets ? offsets[e] : (int64_t)e * npe;
-
-  // net 0 <- component c of the element's control points
-  float mn = INFINITY, mx = -INFINITY;
-  for (int d = lane; d < npe; d += 64)
-  {
-    const float v = values[(int64_t)ctrl_idx[off + d] * 3 + c];
-    nets[c * NPE + d] = v;
-    mn = fminf (mn, v);
-    mx = fmaxf (mx, v);
-  }
-  const int32_t kmn = wave_reduce_min (float_key (mn)), kmx = wave_reduce_max (float_key (mx));
-  if (lane == 0)   // buffer 0: the first split (count 1) writes buffer 1, and count 2 writes buffer 0 only
-  {                // after every wavefront has passed count 1's barrier, so after these reads
-    xch[0][c][0] = key_float (kmn);
-    xch[0][c][1] = key_float (kmx);
+    for (int c = 0; c < 3; ++c) nets[c * CS + d] = values[g + c];
   }
   __syncthreads ();
-  float my_box[6], my_ref[6], my_meas = -INFINITY;
-  {
-    float b0[6];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      b0[2 * d] = xch[0][d][0];
-      b0[2 * d + 1] = xch[0][d][1];
-    }
-#pragma unroll
-    for (int q = 0; q < 6; ++q) my_box[q] = b0[q];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      my_ref[d] = 0.f;
-      my_ref[3 + d] = 1.f;
-    }
-    if (lane == 0) my_meas = box_measure (b0);
-  }
+  const int group = threadIdx.x / G, n_groups = 64 * WAVES / G, gl = threadIdx.x % G;
+  split_level<P, 0> (nets, hulls, group, n_groups, gl);
+  __syncthreads ();
+  split_level<P, 1> (nets, hulls, group, n_groups, gl);
+  __syncthreads ();
+  split_level<P, 2> (nets, hulls, group, n_groups, gl);
+  __syncthreads ();
+  split_level<P, 3> (nets, hulls, group, n_groups, gl);
+  __syncthreads ();
+  split_level<P, 4> (nets, hulls, group, n_groups, gl);
+  __syncthreads ();
+  if (threadIdx.x >= 64) return;
 
-  for (int count = 1; count <= kSplitBoxes - 1; ++count)
-  {
-    int max_id = 0;
-    {
-      const float m0 = __int_as_float (__builtin_amdgcn_readfirstlane (__float_as_int (my_meas)));
-      if (m0 == m0)
-      {
-        const int32_t cand = (lane < count && my_meas == my_meas) ? float_key (my_meas) : INT32_MIN;
-        const int32_t M = wave_reduce_max (cand);
-        const uint64_t hit = __ballot (lane < count && cand == M);
-        max_id = __ffsll ((unsigned long long)hit) - 1;
-      }
-    }
-    float sr[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) sr[q] = __int_as_float (__builtin_amdgcn_readlane (__float_as_int (my_ref[q]), max_id));
-    int axis = 0;
-    float maxlen = sr[3] - sr[0];
-    for (int d = 1; d < 3; ++d)
-    {
-      const float len = sr[3 + d] - sr[d];
-      if (len > maxlen)
-      {
-        axis = d;
-        maxlen = len;
-      }
-    }
-    const float split_pt = sr[axis] * (1.0f - 0.5f) + sr[3 + axis] * 0.5f;
-    if (lane == count)
-    {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_ref[q] = (q == axis) ? split_pt : sr[q];
-    }
-    if (lane == max_id)
-    {
-#pragma unroll
-      for (int d = 0; d < 3; ++d)
-        if (d == axis) my_ref[3 + d] = split_pt;
-    }
-    float *mom = nets + (max_id * 3 + c) * NPE;
-    float *dau = nets + (count * 3 + c) * NPE;
-    float lo_a = INFINITY, hi_a = -INFINITY, lo_b = INFINITY, hi_b = -INFINITY;
-    if (p == PMAX)
-      split_lines_comp<PMAX> (mom, dau, axis, lane, lo_a, hi_a, lo_b, hi_b);
-    else
-      switch (p)   // mixed-order meshes
-      {
-      case 1: split_lines_comp<1> (mom, dau, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      case 2: split_lines_comp<(PMAX >= 2 ? 2 : 1)> (mom, dau, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      case 3: split_lines_comp<(PMAX >= 3 ? 3 : 1)> (mom, dau, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      default: split_lines_comp<(PMAX >= 4 ? 4 : 1)> (mom, dau, axis, lane, lo_a, hi_a, lo_b, hi_b); break;
-      }
-    // the lanes' hulls are never NaN (fminf / fmaxf from +-inf skip NaN values): integer keys reduce them
-    const int32_t klo_a = wave_reduce_min (float_key (lo_a)), khi_a = wave_reduce_max (float_key (hi_a));
-    const int32_t klo_b = wave_reduce_min (float_key (lo_b)), khi_b = wave_reduce_max (float_key (hi_b));
-    const int par = count & 1;
-    if (lane == 0)
-    {
-      xch[par][c][0] = key_float (klo_a);
-      xch[par][c][1] = key_float (khi_a);
-      xch[par][c][2] = key_float (klo_b);
-      xch[par][c][3] = key_float (khi_b);
-    }
-    __syncthreads ();
-    float ba[6], bb[6];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      ba[2 * d] = xch[par][d][0];
-      ba[2 * d + 1] = xch[par][d][1];
-      bb[2 * d] = xch[par][d][2];
-      bb[2 * d + 1] = xch[par][d][3];
-    }
-    if (lane == max_id)
-    {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_box[q] = ba[q];
-      my_meas = box_measure (ba);
-    }
-    if (lane == count)
-    {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) my_box[q] = bb[q];
-      my_meas = box_measure (bb);
-    }
-  }
-
-  if (c == 0 && lane < kSplitBoxes)
+  // lane h (1..63): key of the measure of the box with heap index h (the element, h 1, is split first whatever it is)
+  float node_meas;
   {
     float b[6];
-    for (int q = 0; q < 6; ++q) b[q] = my_box[q];
-    const float s = (float)1.000001;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-      float lo = b[2 * d], hi = b[2 * d + 1];
-      if (!(lo > hi))
-      {
-        const float cc = 0.5f * (lo + hi);
-        const float delta = s * 0.5f * (hi - lo);
-        const float v0 = cc - delta, v1 = cc + delta;
-        lo = fminf (lo, v0);
-        hi = fmaxf (hi, v0);
-        lo = fminf (lo, v1);
-        hi = fmaxf (hi, v1);
-      }
-      b[2 * d] = lo;
-      b[2 * d + 1] = hi;
-    }
-    const int64_t k = (int64_t)e * kSplitBoxes + lane;
-    for (int q = 0; q < 6; ++q)
-    {
-      out_aabbs[6 * k + q] = b[q];
-      out_subrefs[6 * k + q] = my_ref[q];
-    }
-    out_prims[k] = e;
+    for (int q = 0; q < 6; ++q) b[q] = hulls[6 * lane + q];
+    node_meas = box_measure (b);
   }
-  __syncthreads ();   // the next element rewrites the nets and the exchange buffers
+  const int64_t k0 = (int64_t)e * kSplitBoxes;
+  if (!split_ranked<P> (nets, hulls, extra, node_meas, lane, k0, out_aabbs, out_subrefs))
+    split_sequential<P> (nets, hulls, node_meas, lane, k0, out_aabbs, out_subrefs);
+  if (lane < kSplitBoxes) out_prims[k0 + lane] = e;
+}
+
+template <int PMAX, int WAVES>
+__global__ void __launch_bounds__ (64 * WAVES) k_split (const int32_t *__restrict__ ctrl_idx, const float *__restrict__ values,
+                                                        const int32_t *__restrict__ orders,
+                                                        const int64_t *__restrict__ offsets, int n_el,
+                                                        float *__restrict__ out_aabbs, int32_t *__restrict__ out_prims,
+                                                        float *__restrict__ out_subrefs)
+{
+  __shared__ __attribute__ ((aligned (16))) float nets[kSplitNets * 3 * SplitOrd<PMAX>::CS];
+  __shared__ float hulls[64 * 6], extra[2 * kSplitExtras * 6];
+  const int e = blockIdx.x;
+  if (e >= n_el) return;
+  const int64_t off = offsets ? offsets[e] : (int64_t)e * SplitOrd<PMAX>::NPE;
+#define DRX_SPLIT_ELEMENT(P) split_element<P, WAVES> (ctrl_idx, values, off, e, nets, hulls, extra, out_aabbs, out_prims, out_subrefs)
+  if constexpr (PMAX == DRX_MAX_MIXED_ORDER)
+  {
+    switch (orders ? orders[e] : PMAX)   // mixed-order meshes
+    {
+    case 1: DRX_SPLIT_ELEMENT (1); break;
+    case 2: DRX_SPLIT_ELEMENT (2); break;
+    case 3: DRX_SPLIT_ELEMENT (3); break;
+    default: DRX_SPLIT_ELEMENT (4); break;
+    }
   }
+  else
+    DRX_SPLIT_ELEMENT (PMAX);
+#undef DRX_SPLIT_ELEMENT
 }
 
 // =============================================================================================
@@ -1010,25 +1006,23 @@ int drx_bvh_split_elements (const int32_t *ctrl_idx, const float *values, const 
   if (pmax < 1 || pmax > DRX_MAX_ORDER)
     return fail (DRX_ERR_ARG, "drx_bvh_split_elements: order %d outside 1..%d", order, DRX_MAX_ORDER);
   hipStream_t st = as_stream (stream);
-  float *gnets = nullptr;
-  const int gn_blocks = n_el < kSplitGlobalBlocks ? n_el : kSplitGlobalBlocks;
-  if (pmax >= 7)
-  {
-    const size_t npe = (size_t)(pmax + 1) * (pmax + 1) * (pmax + 1);
-    gnets = (float *)arena (SLOT_TREE, sizeof (float) * kSplitBoxes * 3 * npe * gn_blocks, st);
-    if (!gnets) return DRX_ERR_HIP;
-  }
+#define DRX_SPLIT_GO(P, W)                                                                                       \
+  hipLaunchKernelGGL ((k_split<P, W>), dim3 (n_el), dim3 (64 * W), 0, st, ctrl_idx, values, orders, offsets, n_el, \
+                      out_aabbs, out_prims, out_subrefs)
   switch (pmax)
   {
-  case 1: hipLaunchKernelGGL (k_split<1>, dim3 (n_el), dim3 (64), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs); break;
-  case 2: hipLaunchKernelGGL (k_split<2>, dim3 (n_el), dim3 (64), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs); break;
-  case 3: hipLaunchKernelGGL (k_split<3>, dim3 (n_el), dim3 (64), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs); break;
-  case 4: hipLaunchKernelGGL ((k_split_cw<4, false>), dim3 (n_el), dim3 (192), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs, nullptr); break;
-  case 5: hipLaunchKernelGGL ((k_split_cw<5, false>), dim3 (n_el), dim3 (192), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs, nullptr); break;
-  case 6: hipLaunchKernelGGL ((k_split_cw<6, false>), dim3 (n_el), dim3 (192), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs, nullptr); break;
-  case 7: hipLaunchKernelGGL ((k_split_cw<7, true>), dim3 (gn_blocks), dim3 (192), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs, gnets); break;
-  default: hipLaunchKernelGGL ((k_split_cw<8, true>), dim3 (gn_blocks), dim3 (192), 0, st, ctrl_idx, values, orders, offsets, order, n_el, out_aabbs, out_prims, out_subrefs, gnets); break;
+  // wavefronts per element: order 2 one (64,000 elements 249 us, two 260), order 3 four (262,144 elements
+  // 1.08 ms, two 1.15, one 1.31), order 4 four (64,000 elements 672 us, two 789)
+  case 1: DRX_SPLIT_GO (1, 1); break;
+  case 2: DRX_SPLIT_GO (2, 1); break;
+  case 3: DRX_SPLIT_GO (3, 4); break;
+  case 4: DRX_SPLIT_GO (4, 4); break;
+  case 5: DRX_SPLIT_GO (5, 4); break;
+  case 6: DRX_SPLIT_GO (6, 8); break;
+  case 7: DRX_SPLIT_GO (7, 8); break;
+  default: DRX_SPLIT_GO (8, 8); break;
   }
+#undef DRX_SPLIT_GO
   DRX_LAUNCH_CHECK ();
   return DRX_OK;
 }
