@@ -207,6 +207,48 @@ __global__ void __launch_bounds__ (kScanBlock) k_scan_down (const int32_t *in, i
   }
 }
 
+// Small arrays (the digit counts of a sort of up to half a million keys, the flags of small frames): one block walks the
+// array with a carry, one launch instead of three (8,704 counts: 10 us against 12 us and two launches).  total -> *total.
+constexpr int kScanSmallBlock = 1024, kScanSmallItems = 8, kScanSmallMax = 4 * kScanSmallBlock * kScanSmallItems;
+
+__global__ void __launch_bounds__ (kScanSmallBlock) k_scan_small (const int32_t *in, int32_t *out, int32_t n, int32_t *total)
+{
+  __shared__ int32_t wsum[kScanSmallBlock / 64];
+  const int w = threadIdx.x >> 6;
+  int32_t carry = 0;
+  for (int32_t base = 0; base < n; base += kScanSmallBlock * kScanSmallItems)
+  {
+    const int32_t i0 = base + (int32_t)threadIdx.x * kScanSmallItems;
+    int32_t v[kScanSmallItems], s = 0;
+#pragma unroll
+    for (int k = 0; k < kScanSmallItems; ++k)
+    {
+      v[k] = i0 + k < n ? in[i0 + k] : 0;
+      s += v[k];
+    }
+    const int32_t incl = wave_scan_incl_add (s);
+    if ((threadIdx.x & 63) == 63) wsum[w] = incl;
+    __syncthreads ();
+    int32_t before = carry;
+#pragma unroll
+    for (int q = 0; q < kScanSmallBlock / 64; ++q)
+    {
+      const int32_t t = wsum[q];
+      carry += t;
+      before += q < w ? t : 0;
+    }
+    int32_t at = before + incl - s;
+#pragma unroll
+    for (int k = 0; k < kScanSmallItems; ++k)
+    {
+      if (i0 + k < n) out[i0 + k] = at;
+      at += v[k];
+    }
+    __syncthreads ();
+  }
+  if (threadIdx.x == 0) *total = carry;
+}
+
 int32_t scan_sums_len (int32_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
 int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *total_host, hipStream_t st, int32_t *sums)
@@ -219,9 +261,14 @@ int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *tot
   const int32_t nb = (n + kScanTile - 1) / kScanTile;
   if (!sums) sums = (int32_t *)arena (SLOT_SCAN, sizeof (int32_t) * (nb + 1), st);
   if (!sums) return DRX_ERR_HIP;
-  hipLaunchKernelGGL (k_scan_reduce, dim3 (nb), dim3 (kScanBlock), 0, st, in, n, sums);
-  hipLaunchKernelGGL (k_scan_sums, dim3 (1), dim3 (kScanBlock), 0, st, sums, nb);
-  hipLaunchKernelGGL (k_scan_down, dim3 (nb), dim3 (kScanBlock), 0, st, in, out, n, sums);
+  if (n <= kScanSmallMax)
+    hipLaunchKernelGGL (k_scan_small, dim3 (1), dim3 (kScanSmallBlock), 0, st, in, out, n, sums + nb);
+  else
+  {
+    hipLaunchKernelGGL (k_scan_reduce, dim3 (nb), dim3 (kScanBlock), 0, st, in, n, sums);
+    hipLaunchKernelGGL (k_scan_sums, dim3 (1), dim3 (kScanBlock), 0, st, sums, nb);
+    hipLaunchKernelGGL (k_scan_down, dim3 (nb), dim3 (kScanBlock), 0, st, in, out, n, sums);
+  }
   DRX_LAUNCH_CHECK ();
   if (total_host)
   {
