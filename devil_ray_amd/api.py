@@ -70,6 +70,8 @@ class BVH:
         self.qnodes = None          # compact traversal nodes (drx_bvh_quantize) + exact leaf boxes + grid
         self.leaf_boxes = None
         self.qgrid = np.zeros(6, np.float32)
+        self.entry_cells = None     # entry cells of the binary walk (drx_bvh_entry_cells)
+        self.entry_bits = np.zeros(3, np.int32)
         self.use_wide = True
         self.use_starts = True
         self.use_qnodes = True
@@ -95,6 +97,9 @@ class BVH:
             v.leaf_boxes = self.leaf_boxes.data_ptr()
             for q in range(6):
                 v.qgrid[q] = float(self.qgrid[q])
+            if self.entry_cells is not None:
+                v.entry_cells = self.entry_cells.data_ptr()
+                v.entry_bits[:] = [int(b) for b in self.entry_bits]
         return v
 
     def quantize(self) -> None:
@@ -109,6 +114,16 @@ class BVH:
                                          C.cast(grid, C.c_void_p), _stream()),
                 "drx_bvh_quantize")
         self.qgrid = np.array(list(grid), np.float32)
+
+    def compute_entry_cells(self) -> None:
+        """Entry cells of the binary walk over the compact nodes (drx_bvh_entry_cells)."""
+        b = np.ascontiguousarray(self.bounds, np.float32)
+        n = L.lib().drx_bvh_entry_bits(self.n_leaves, b.ctypes.data, self.entry_bits.ctypes.data)
+        cells = torch.empty(int(n) * 4, dtype=torch.int32, device=_dev())
+        v = self.view()
+        L.check(L.lib().drx_bvh_entry_cells(C.byref(v), self.entry_bits.ctypes.data, _ptr(cells), _stream()),
+                "drx_bvh_entry_cells")
+        self.entry_cells = cells
 
     def compute_leaf_starts(self, mesh_view: L.DrxMesh) -> None:
         """Per-leaf Newton start maps (drx_bvh_leaf_starts) from the geometry the BVH was built on."""
@@ -305,6 +320,7 @@ class UnstructuredMesh:
             bvh.pack_leaves()
             bvh.compute_leaf_starts(self.gf.view())
             bvh.quantize()
+            bvh.compute_entry_cells()
             if bvh.n_leaves <= WIDE_EAGER_MAX_LEAVES:
                 bvh.widen()   # small BVHs: the automatic walk of a render may take the wave walk
             self._bvh = bvh

@@ -194,6 +194,10 @@ template <class ElemT> BVH &UnstructuredMesh<ElemT>::get_bvh ()
     drx_check (drx_bvh_quantize (&v, m_bvh.m_qnodes.get_device_ptr (), m_bvh.m_leaf_boxes.get_device_ptr (),
                                  m_bvh.m_qgrid, nullptr),
                "drx_bvh_quantize");
+    v = bvh_view ();
+    m_bvh.m_entry_cells.resize (4 * (size_t)drx_bvh_entry_bits (v.n_leaves, v.bounds, m_bvh.m_entry_bits));
+    drx_check (drx_bvh_entry_cells (&v, m_bvh.m_entry_bits, m_bvh.m_entry_cells.get_device_ptr (), nullptr),
+               "drx_bvh_entry_cells");
     // the 8-wide copy, read only by the wave walk that the automatic choice takes for small BVHs
     if (m_bvh.m_leaf_nodes.size () <= (size_t (1) << 16))
     {
@@ -229,6 +233,11 @@ template <class ElemT> drx_bvh UnstructuredMesh<ElemT>::bvh_view ()
     v.qnodes = m_bvh.m_qnodes.get_device_ptr_const ();
     v.leaf_boxes = m_bvh.m_leaf_boxes.get_device_ptr_const ();
     for (int q = 0; q < 6; ++q) v.qgrid[q] = m_bvh.m_qgrid[q];
+    if (m_is_constructed)
+    {
+      v.entry_cells = m_bvh.m_entry_cells.get_device_ptr_const ();
+      for (int d = 0; d < 3; ++d) v.entry_bits[d] = m_bvh.m_entry_bits[d];
+    }
   }
   return v;
 }

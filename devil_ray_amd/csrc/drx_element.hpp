@@ -464,6 +464,8 @@ struct LocateCfg
   const uint4 *qnodes;      // optional compact inner nodes, 2 uint4 each (then leaf_boxes and the grid are set)
   const float4 *leaf_boxes; // with qnodes: exact leaf boxes, 2 float4 each
   float q_org[3], q_inv[3]; // with qnodes: grid origin and cells per unit length
+  const uint4 *entry;       // with qnodes, optional: entry cells (drx_bvh_entry_cells)
+  int entry_bits[3];        // with entry: log2 of the cells per axis
   const float4 *wide;       // 8-wide nodes, 16 float4 each (nullptr: binary traversal)
   const float4 *leaves;     // packed leaves, 2 float4 each
   const float4 *starts;     // optional Newton start maps, 3 float4 per leaf (drx_bvh_leaf_starts)
@@ -730,6 +732,29 @@ __device__ __forceinline__ const float *stage_element (const LocateCfg &cfg, int
   return slot >= 0 ? stage + slot * F4 * 4 : g;
 }
 
+// Starts a lane's depth-first walk for point pt: at the root or, when the BVH has entry cells, at the subtrees
+// listed for the point's cell (the first one in cur, the others on the stack above kBarrier).  They hold every
+// leaf whose box can contain a point of the cell, in depth-first order, so the candidates and their order are the
+// root walk's.  A NaN coordinate has cell 0 and no leaf box contains it.
+__device__ __forceinline__ void walk_start (const LocateCfg &cfg, TravStack &todo, const float pt[3], int &cur, int &sp)
+{
+  todo.set (0, kBarrier);
+  sp = 0;
+  cur = 0;
+  if (cfg.entry)
+  {
+    const int bx = cfg.entry_bits[0], by = cfg.entry_bits[1], bz = cfg.entry_bits[2];
+    const uint32_t cx = grid_cell (pt[0], cfg.q_org[0], cfg.q_inv[0]) >> (16 - bx),
+                   cy = grid_cell (pt[1], cfg.q_org[1], cfg.q_inv[1]) >> (16 - by),
+                   cz = grid_cell (pt[2], cfg.q_org[2], cfg.q_inv[2]) >> (16 - bz);
+    const uint4 e = cfg.entry[(((size_t)cz << by | cy) << bx) | cx];
+    cur = (int)e.x;
+    if ((int)e.w != kBarrier) todo.set (++sp, (int)e.w);
+    if ((int)e.z != kBarrier) todo.set (++sp, (int)e.z);
+    if ((int)e.y != kBarrier) todo.set (++sp, (int)e.y);
+  }
+}
+
 constexpr int kWalkDone = -1, kWalkOverflow = -2;
 
 // DeviceMesh::locate's traversal (device_mesh.hpp:262-320) from the state (cur, sp) to the next candidate
@@ -825,8 +850,8 @@ __device__ __forceinline__ int next_candidate_leaf (const LocateCfg &cfg, TravSt
     if (!compact) break;
     // the cell ranges are conservative: the leaf's exact box (dray's child-box test) decides
     const float4 b0 = cfg.leaf_boxes[2 * (int64_t)leaf], b1 = cfg.leaf_boxes[2 * (int64_t)leaf + 1];
-    const bool in = !(pt[0] < b0.x) && !(pt[1] < b0.y) && !(pt[2] < b0.z) && !(pt[0] > b0.w) && !(pt[1] > b1.x) &&
-                    !(pt[2] > b1.y);
+    // (a NaN coordinate, whose cell 0 lies outside every box's cell range, is in no box)
+    const bool in = pt[0] >= b0.x && pt[1] >= b0.y && pt[2] >= b0.z && pt[0] <= b0.w && pt[1] <= b1.x && pt[2] <= b1.y;
     if (in) break;
     cur = todo.get (sp);
     --sp;
@@ -838,7 +863,7 @@ __device__ __forceinline__ int next_candidate_leaf (const LocateCfg &cfg, TravSt
 // the point is in both; the first accepted candidate wins.
 //
 // Resumable form, one candidate per call: cur / sp carry this lane's depth-first state between calls
-// (start a search with cur = 0, sp = 0 and kBarrier in stack entry 0).  The lane walks inner nodes until
+// (start a search with walk_start).  The lane walks inner nodes until
 // it holds a leaf (lanes that get there early wait, so the Newton solve runs with the wave converged),
 // then tests that one candidate.  Returns 1 if it was accepted (ref, cell set), 0 if it was rejected (the
 // state then holds the next stack entry: call again with the same point), -1 when the search is
@@ -891,8 +916,8 @@ template <int P, bool POLISH>
 __device__ __forceinline__ int locate_point (const LocateCfg &cfg, TravStack &todo, const float pt[3], float ref[3],
                                              LocateStats &st, bool &overflow)
 {
-  int cur = 0, sp = 0, cell = -1;
-  todo.set (0, kBarrier);
+  int cur, sp, cell = -1;
+  walk_start (cfg, todo, pt, cur, sp);
   for (;;)
   {
     const int r = locate_point_step<P, POLISH> (cfg, todo, pt, ref, st, overflow, cur, sp, cell);

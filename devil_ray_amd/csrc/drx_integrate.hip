@@ -266,12 +266,7 @@ __global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) 
       if constexpr (LEARNED)
       {
         // one candidate per iteration as in the plain walks; every lane joins the wavefront's MLP round
-        if (alive && !resume)
-        {
-          tcur = 0;
-          tsp = 0;
-          todo.set (0, kBarrier);
-        }
+        if (alive && !resume) walk_start (a.cfg, todo, pt, tcur, tsp);
         int c = -1;
         const int r = locate_point_mlp_step<P, POLISH> (a.cfg, todo, pt, ref, st, overflow, alive, tcur, tsp, c, a.net,
                                                         a.budget, mlp_x + wv * 64 * mlp::IN_PAD, mlp_y + wv * 64 * 4);
@@ -286,9 +281,10 @@ __global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) 
       {
         if (!resume)
         {
-          tcur = 0;
-          tsp = 0;
-          if constexpr (MODE != 1) todo.set (0, kBarrier);
+          if constexpr (MODE == 1)
+            tcur = tsp = 0;
+          else
+            walk_start (a.cfg, todo, pt, tcur, tsp);
           if constexpr (GUIDED)
           {
             given.cell = -1;

@@ -64,8 +64,7 @@ __device__ __forceinline__ bool try_element_learned_mixed (const LocateCfg &cfg,
   }
 }
 
-// One candidate per call, resumable like locate_point_step (start a point with cur = 0, sp = 0 and kBarrier
-// in stack entry 0).  Every lane of the wavefront calls it, with have == false when it holds no point,
+// One candidate per call, resumable like locate_point_step (start a point with walk_start).  Every lane of the wavefront calls it, with have == false when it holds no point,
 // because the MLP round is wavefront-wide.  Returns 1 if the candidate was accepted (ref, cell set), 0 if it
 // was rejected (call again with the same point), -1 when the search is exhausted or the stack would
 // overflow (overflow set) or the lane holds no point.

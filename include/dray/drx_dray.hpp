@@ -167,6 +167,8 @@ struct BVH
   Array<uint32> m_qnodes;         // compact traversal nodes (drx_bvh_quantize)
   Array<float32> m_leaf_boxes;    // exact leaf boxes for the compact walk
   float32 m_qgrid[6] = { 0, 0, 0, 0, 0, 0 };
+  Array<uint32> m_entry_cells;    // entry cells of the binary walk (drx_bvh_entry_cells)
+  int32 m_entry_bits[3] = { 0, 0, 0 };
   Array<float32> m_wide_nodes;
 };
 

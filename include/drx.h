@@ -108,7 +108,9 @@ typedef struct drx_bvh
                                  binary walks use them, with leaf_boxes and qgrid, when set */
   const float *leaf_boxes;    /* with qnodes: 8 floats per leaf, its exact box {lo xyz, hi x, hi yz, 0, 0} */
   float qgrid[6];             /* with qnodes: grid origin xyz, grid cells per unit length xyz */
-} drx_bvh;
+  const uint32_t *entry_cells;/* optional, with qnodes: entry cells of the binary walk (drx_bvh_entry_cells) */
+  int32_t entry_bits[3];      /* with entry_cells: 2^bits cells along x, y, z */
+} drx_bvh;                    /* zero the struct before filling it in: members left out are then not used */
 
 /* Location (location.hpp:16-21): {int32 cell (-1 = not found), float ref[3]} = 16 bytes. */
 /* Ray (ray.hpp:20-28): {float dir[3], near, orig[3], far; int32 pixel_id} = 36 bytes.   */
@@ -298,6 +300,14 @@ int drx_bvh_leaf_starts (const drx_mesh *mesh, const drx_bvh *bvh, float *out_le
  * per leaf) before Newton, so the candidates and their order are dray's.  out_grid (host, 6 floats):
  * origin xyz, cells per unit xyz; copy it into drx_bvh.qgrid.  Needs inner_nodes, n_leaves, bounds. */
 int drx_bvh_quantize (const drx_bvh *bvh, uint32_t *out_qnodes, float *out_leaf_boxes, float *out_grid, void *stream);
+/* Entry cells of the binary walk (no dray counterpart; dray's walk starts at the root for every point,
+ * device_mesh.hpp:262-320).  The grid of drx_bvh_quantize is cut into 2^bits[d] cells per axis; each cell holds up
+ * to 4 child codes of the compact nodes, in dray's depth-first order, whose subtrees hold every leaf that a point of
+ * the cell can reach (-2000000000: unused).  A walk that starts from its point's cell visits the same leaves in
+ * the same order as one that starts at the root.  drx_bvh_entry_bits (host) picks bits for a BVH of n_leaves over
+ * bounds and returns the number of cells; out_cells: 4 words per cell.  Needs n_leaves, qnodes, qgrid. */
+int64_t drx_bvh_entry_bits (int32_t n_leaves, const float *bounds6, int32_t *out_bits);
+int drx_bvh_entry_cells (const drx_bvh *bvh, const int32_t *bits, uint32_t *out_cells, void *stream);
 /* 8-wide traversal copy of the binary BVH: children in binary left-to-right order, exact float boxes,
  * so traversal visits the same candidate leaves in the same order as dray's binary depth-first walk.
  * Node = 64 floats: lo_x[8] lo_y[8] lo_z[8] hi_x[8] hi_y[8] hi_z[8] child[8] (int32 bits) pad[8].
