@@ -163,8 +163,8 @@ def main() -> int:
     achieved_gbs = located_per_frame * bytes_per_sample / (k_ms * 1e-3) / 1e9
     walk = int(st.walk)   # the walk the library ran (the automatic choice depends on the frame's size)
     pol, shade = 'true' if args.polish else 'false', 2 if fp64_field else 0
-    # walk 5: the sample-parallel kernel the library takes for frames of few rays per SIMD
-    kernel_name = (f"k_integrate_split<{p},{pol},{shade}>" if walk == 5 else f"k_integrate<{p},{pol},{walk},{shade}>")
+    # walk 5: the sample-parallel kernel (these frames have well over 32 rays per element column)
+    kernel_name = (f"k_integrate_binned<{p},{pol},{shade}>" if walk == 5 else f"k_integrate<{p},{pol},{walk},{shade}>")
 
     out = {
         "metric": "located samples/s (volume render; also Mrays/s)",

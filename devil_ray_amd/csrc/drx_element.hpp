@@ -18,6 +18,10 @@ namespace drx
 #define DRX_EVAL_ROTATE_MIN_ORDER 4   // orders >= this rotate the w-weight arrays per slab instead of selecting
 #endif                                // by slab index (measured: faster at order 4, slower at order 3)
 
+// Wave-uniform reads through the constant address space become scalar loads.
+typedef const float __attribute__ ((address_space (4))) cfloat;
+typedef const double __attribute__ ((address_space (4))) cdouble;
+
 template <int P> struct Ord
 {
   static constexpr int N1 = P + 1;
@@ -69,8 +73,9 @@ __device__ __forceinline__ T pick (const T arr[N], int k)
 
 // phi(x) - origin and the Jacobian J[c][a] = d phi_c / d x_a of a packed geometry block.
 // The w-slabs are walked by a rolled loop so that only one slab of control points is live at a time.
-template <int P, typename T>
-__device__ __forceinline__ void eval_geom (const float *__restrict__ g, const T x[3], T y[3], T J[3][3])
+// G: const float * (a lane's own element) or cfloat * (one element for the whole wavefront).
+template <int P, typename T, typename G>
+__device__ __forceinline__ void eval_geom (G __restrict__ g, const T x[3], T y[3], T J[3][3])
 {
   constexpr int N1 = Ord<P>::N1, NP = Ord<P>::NP;
   T Bu[N1], dBu[N1], Bv[N1], dBv[N1], Bw[N1], dBw[N1];
@@ -78,7 +83,7 @@ __device__ __forceinline__ void eval_geom (const float *__restrict__ g, const T 
   bernstein<P, T> (x[1], Bv, dBv);
   bernstein<P, T> (x[2], Bw, dBw);
   T val[3] = { 0, 0, 0 }, du[3] = { 0, 0, 0 }, dv[3] = { 0, 0, 0 }, dw[3] = { 0, 0, 0 };
-  const float *X = g + 4;
+  const G X = g + 4;
 #pragma unroll DRX_EVAL_UNROLL_K
   for (int k = 0; k < N1; ++k)
   {
@@ -101,7 +106,7 @@ __device__ __forceinline__ void eval_geom (const float *__restrict__ g, const T 
       bw = pick<N1, T> (Bw, k);
       dbw = pick<N1, T> (dBw, k);
     }
-    const float *slab = X + N1 * N1 * k;
+    const G slab = X + N1 * N1 * k;
 #pragma unroll
     for (int j = 0; j < N1; ++j)
     {
@@ -187,11 +192,12 @@ __device__ __forceinline__ void eval_geom_regs (const float (&C)[3][Ord<P>::NPE]
   }
 }
 
-// Scalar field value at reference point x; FT = float, or double for an FP64 field (evaluated in double
+// Scalar field value at reference point x; F points to float, or to double for an FP64 field (evaluated in double
 // at the float32 reference point).
-template <int P, typename FT = float>
-__device__ __forceinline__ FT eval_scalar (const FT *__restrict__ f, const float x[3])
+template <int P, typename F>
+__device__ __forceinline__ auto eval_scalar (F __restrict__ f, const float x[3])
 {
+  using FT = decltype (+f[0]);
   constexpr int N1 = Ord<P>::N1;
   FT Bu[N1], dBu[N1], Bv[N1], dBv[N1], Bw[N1], dBw[N1];
   bernstein<P, FT> ((FT)x[0], Bu, dBu);
@@ -217,8 +223,8 @@ __device__ __forceinline__ FT eval_scalar (const FT *__restrict__ f, const float
 }
 
 // Scalar value and reference-space gradient (for lit shading).
-template <int P>
-__device__ __forceinline__ float eval_scalar_d (const float *__restrict__ f, const float x[3], float d[3])
+template <int P, typename F>
+__device__ __forceinline__ float eval_scalar_d (F __restrict__ f, const float x[3], float d[3])
 {
   constexpr int N1 = Ord<P>::N1;
   float Bu[N1], dBu[N1], Bv[N1], dBv[N1], Bw[N1], dBw[N1];
@@ -352,8 +358,8 @@ struct NewtonOut
 // steps; each clamps x into [0,1], evaluates phi and J, solves J dx = target - phi by LUP, x += dx;
 // converged when |x - prev|inf < 1e-4; accepted when converged and x in [-1e-4, 1+1e-4]^3.
 // `t` is the target relative to the block's origin.
-template <int P, bool REGS>
-__device__ __forceinline__ bool newton_f32 (const float *__restrict__ g, const float t[3], float x[3], NewtonOut &no,
+template <int P, bool REGS, typename G>
+__device__ __forceinline__ bool newton_f32 (G __restrict__ g, const float t[3], float x[3], NewtonOut &no,
                                             bool want_cond, int max_steps = 20)
 {
   // REGS: the element's control points are loaded once into registers and reused by every iteration
@@ -490,13 +496,24 @@ struct LocateStats
   int fallbacks;   // learned-start Newton runs that did not converge and were redone from the plain start
 };
 
-template <int P, bool POLISH>
+// UNI: every active lane tests the same element (g wave-uniform), read by scalar loads.
+template <int P, bool POLISH, bool UNI = false>
 __device__ __forceinline__ bool try_element_at (const LocateCfg &cfg, const float *g, const float pt[3], float x[3],
                                                 LocateStats &st)
 {
-  const float t[3] = { pt[0] - g[0], pt[1] - g[1], pt[2] - g[2] };
   NewtonOut no;
-  const bool found = newton_f32<P, (P <= DRX_REG_ELEMENT_MAX_ORDER)> (g, t, x, no, POLISH);
+  bool found;
+  if constexpr (UNI)
+  {
+    cfloat *gu = (cfloat *)g;
+    const float t[3] = { pt[0] - gu[0], pt[1] - gu[1], pt[2] - gu[2] };
+    found = newton_f32<P, false> (gu, t, x, no, POLISH);
+  }
+  else
+  {
+    const float t[3] = { pt[0] - g[0], pt[1] - g[1], pt[2] - g[2] };
+    found = newton_f32<P, (P <= DRX_REG_ELEMENT_MAX_ORDER)> (g, t, x, no, POLISH);
+  }
   st.newton += no.steps;
   st.candidates += 1;
   if constexpr (POLISH)
@@ -514,17 +531,17 @@ __device__ __forceinline__ bool try_element_at (const LocateCfg &cfg, const floa
 }
 
 // Runtime-order dispatch for mixed meshes.
-template <bool POLISH>
+template <bool POLISH, bool UNI = false>
 __device__ __forceinline__ bool try_element_mixed (const LocateCfg &cfg, int el, const float pt[3], float x[3],
                                                    LocateStats &st)
 {
   const float *g = cfg.mesh + cfg.offsets[el];
   switch (cfg.orders[el])
   {
-  case 1: return try_element_at<1, POLISH> (cfg, g, pt, x, st);
-  case 2: return try_element_at<2, POLISH> (cfg, g, pt, x, st);
-  case 3: return try_element_at<3, POLISH> (cfg, g, pt, x, st);
-  default: return try_element_at<4, POLISH> (cfg, g, pt, x, st);
+  case 1: return try_element_at<1, POLISH, UNI> (cfg, g, pt, x, st);
+  case 2: return try_element_at<2, POLISH, UNI> (cfg, g, pt, x, st);
+  case 3: return try_element_at<3, POLISH, UNI> (cfg, g, pt, x, st);
+  default: return try_element_at<4, POLISH, UNI> (cfg, g, pt, x, st);
   }
 }
 
@@ -633,23 +650,21 @@ constexpr int kBarrier = -2000000000;
 
 // Per-lane traversal stack: entries [0, kStackLds) in LDS (entry-major, so the 64 lanes of a wave hit
 // 64 consecutive words), deeper entries in a private array that is touched only by deep traversals.
-struct TravStack
+template <int LDS> struct TravStackOf
 {
-  int32_t *lds;       // kStackLds * blockDim.x words, this lane's column at lds[e * bdim + tid]
+  int32_t *lds;       // LDS * blockDim.x words, this lane's column at lds[e * bdim + tid]
   int bdim, tid;
-  int32_t spill[kStackDepth - kStackLds];
+  int32_t spill[kStackDepth - LDS];
   __device__ __forceinline__ void set (int e, int32_t v)
   {
-    if (e < kStackLds)
+    if (e < LDS)
       lds[e * bdim + tid] = v;
     else
-      spill[e - kStackLds] = v;
+      spill[e - LDS] = v;
   }
-  __device__ __forceinline__ int32_t get (int e) const
-  {
-    return (e < kStackLds) ? lds[e * bdim + tid] : spill[e - kStackLds];
-  }
+  __device__ __forceinline__ int32_t get (int e) const { return (e < LDS) ? lds[e * bdim + tid] : spill[e - LDS]; }
 };
+typedef TravStackOf<kStackLds> TravStack;
 
 // Element staging in LDS: the lanes of a wavefront (rays of one 8x8 tile, or neighbouring query points)
 // mostly test the same few elements.  After traversal each lane holds a candidate; the wavefront takes the
@@ -736,7 +751,8 @@ __device__ __forceinline__ const float *stage_element (const LocateCfg &cfg, int
 // listed for the point's cell (the first one in cur, the others on the stack above kBarrier).  They hold every
 // leaf whose box can contain a point of the cell, in depth-first order, so the candidates and their order are the
 // root walk's.  A NaN coordinate has cell 0 and no leaf box contains it.
-__device__ __forceinline__ void walk_start (const LocateCfg &cfg, TravStack &todo, const float pt[3], int &cur, int &sp)
+template <typename Stack>
+__device__ __forceinline__ void walk_start (const LocateCfg &cfg, Stack &todo, const float pt[3], int &cur, int &sp)
 {
   todo.set (0, kBarrier);
   sp = 0;
@@ -765,7 +781,8 @@ constexpr int kWalkDone = -1, kWalkOverflow = -2;
 // code, its packed record in l0, l1 and its Newton start map in map[] when the BVH has start maps (read
 // together with the exact box over the compact nodes, so a candidate costs one memory round trip),
 // kWalkDone when the stack is exhausted, kWalkOverflow when the 64-entry stack would overflow.
-__device__ __forceinline__ int next_candidate_leaf (const LocateCfg &cfg, TravStack &todo, const float pt[3], int &cur,
+template <typename Stack>
+__device__ __forceinline__ int next_candidate_leaf (const LocateCfg &cfg, Stack &todo, const float pt[3], int &cur,
                                                     int &sp, float4 &l0, float4 &l1, float4 (&map)[3])
 {
   // compact nodes: the point's grid cells, compared with each child box's cell range
@@ -1041,8 +1058,6 @@ __device__ __forceinline__ int locate_any (const LocateCfg &cfg, TravStack &todo
 // full; lanes that accepted drop out of all pending masks and the walk resumes.
 // ---------------------------------------------------------------------------------------------
 constexpr int kWaveStack = 96;   // pending (child, lane mask) entries per wave
-// Wave-uniform node reads go through the constant address space so they become scalar loads.
-typedef const float __attribute__ ((address_space (4))) cfloat;
 constexpr int kCandQ = 4;        // queued candidate leaves per lane
 
 struct WaveScratch

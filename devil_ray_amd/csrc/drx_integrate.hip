@@ -1,5 +1,6 @@
 // Volume::integrate on gfx950: the per-ray march (locate + field / lit shading + LUT + blend, <= 5
 // partials per ray) and partial compaction.
+#include "drx_binned.hpp"
 #include "drx_common.hpp"
 #include "drx_element.hpp"
 #include "drx_locate_mlp.hpp"
@@ -7,6 +8,7 @@
 #include "drx_wave.hpp"
 
 #include <cmath>
+#include <type_traits>
 
 namespace drx
 {
@@ -37,12 +39,21 @@ struct IntegrateArgs
   drx_point_light lights[DRX_MAX_LIGHTS];
 };
 
-template <int P, typename FT = float>
+// A pointer for lanes' own elements (UNI false) or for one element per wavefront, read by scalar loads.
+template <bool UNI, typename T> __device__ __forceinline__ auto element_ptr (const T *p)
+{
+  if constexpr (UNI)
+    return (const T __attribute__ ((address_space (4))) *)p;
+  else
+    return p;
+}
+
+template <int P, bool UNI = false, typename FT>
 __device__ __forceinline__ FT field_at (const IntegrateArgs &a, const FT *field, int cell, const float ref[3])
 {
   if constexpr (P == 0)
   {
-    const FT *f = field + a.field_offsets[cell];
+    const auto f = element_ptr<UNI> (field + a.field_offsets[cell]);
     switch (a.cfg.orders[cell])
     {
     case 1: return eval_scalar<1> (f, ref);
@@ -52,7 +63,7 @@ __device__ __forceinline__ FT field_at (const IntegrateArgs &a, const FT *field,
     }
   }
   else
-    return eval_scalar<P> (field + (int64_t)cell * Ord<P>::FSTRIDE, ref);
+    return eval_scalar<P> (element_ptr<UNI> (field + (int64_t)cell * Ord<P>::FSTRIDE), ref);
 }
 
 // MODE: 0 binary per-lane traversal, 1 8-wide per-lane, 2 8-wide wave-coherent (identical results).
@@ -70,9 +81,8 @@ __device__ __forceinline__ float clamp01f (float v) { return fminf (1.f, fmaxf (
 // physical gradient = ref gradient x J^-1 (three LUP solves, like matrix_inverse), then per light
 // ambient + diffuse + Blinn-Phong specular, gradient flipped toward the light and the half vector
 // (flips persist across lights), channels clamped after each light; alpha <= 0.01 gives zero.
-template <int P>
-__device__ float4 lit_color_at (const IntegrateArgs &a, const float *g, const float *f, const float ref[3],
-                                const Ray &ray)
+template <int P, typename G>
+__device__ __forceinline__ float4 lit_color_at (const IntegrateArgs &a, G g, G f, const float ref[3], const float dir[3])
 {
   float y[3], J[3][3];
   eval_geom<P, float> (g, ref, y, J);
@@ -103,7 +113,7 @@ __device__ float4 lit_color_at (const IntegrateArgs &a, const float *g, const fl
   {
     normalize3 (grad);
     const float wp[3] = { g[0] + y[0], g[1] + y[1], g[2] + y[2] };
-    const float view[3] = { -ray.dir[0], -ray.dir[1], -ray.dir[2] };
+    const float view[3] = { -dir[0], -dir[1], -dir[2] };
     for (int l = 0; l < a.n_lights; ++l)
     {
       const drx_point_light &L = a.lights[l];
@@ -136,24 +146,24 @@ __device__ float4 lit_color_at (const IntegrateArgs &a, const float *g, const fl
   return acc;
 }
 
-template <int P>
-__device__ __forceinline__ float4 lit_color (const IntegrateArgs &a, int cell, const float ref[3], const Ray &ray)
+template <int P, bool UNI = false>
+__device__ __forceinline__ float4 lit_color (const IntegrateArgs &a, int cell, const float ref[3], const float dir[3])
 {
   if constexpr (P == 0)
   {
-    const float *g = a.cfg.mesh + a.cfg.offsets[cell];
-    const float *f = a.field + a.field_offsets[cell];
+    const auto g = element_ptr<UNI> (a.cfg.mesh + a.cfg.offsets[cell]);
+    const auto f = element_ptr<UNI> (a.field + a.field_offsets[cell]);
     switch (a.cfg.orders[cell])
     {
-    case 1: return lit_color_at<1> (a, g, f, ref, ray);
-    case 2: return lit_color_at<2> (a, g, f, ref, ray);
-    case 3: return lit_color_at<3> (a, g, f, ref, ray);
-    default: return lit_color_at<4> (a, g, f, ref, ray);
+    case 1: return lit_color_at<1> (a, g, f, ref, dir);
+    case 2: return lit_color_at<2> (a, g, f, ref, dir);
+    case 3: return lit_color_at<3> (a, g, f, ref, dir);
+    default: return lit_color_at<4> (a, g, f, ref, dir);
     }
   }
   else
-    return lit_color_at<P> (a, a.cfg.mesh + (int64_t)cell * Ord<P>::GSTRIDE, a.field + (int64_t)cell * Ord<P>::FSTRIDE,
-                            ref, ray);
+    return lit_color_at<P> (a, element_ptr<UNI> (a.cfg.mesh + (int64_t)cell * Ord<P>::GSTRIDE),
+                            element_ptr<UNI> (a.field + (int64_t)cell * Ord<P>::FSTRIDE), ref, dir);
 }
 
 #ifndef DRX_INTEGRATE_BLOCK
@@ -171,6 +181,13 @@ constexpr int kWaveWalkMinRaysPerSimd = 48;
 #define DRX_SPLIT_MAX_RAYS_PER_SIMD 300
 #endif
 constexpr int kSplitMaxRaysPerSimd = DRX_SPLIT_MAX_RAYS_PER_SIMD;
+// Of the two sample-parallel kernels, the one that bins candidates by element (k_integrate_binned) takes frames with at
+// least this many active rays per element column (rays / elements^(2/3)); with fewer, 64 neighbouring rays cross too
+// many elements to share them.
+// Measured, binned / per lane, ms at rays per column: 64^3 order 3: 4.17 / 3.15 (6), 4.65 / 4.07 (21), 5.3 / 6.0 (32),
+// 8.6 / 14.0 (93); 40^3 order 4: 4.0 / 3.3 (9), 4.1 / 3.9 (20), 3.3 / 5.1 (46); 56^3 order 2: 3.4 / 3.0 (29); lit 40^3
+// order 3: 1.77 / 1.50 (21), 1.63 / 1.78 (46).
+constexpr double kBinnedMinRaysPerColumn = 32;
 constexpr int kIntWaves = kIntBlock / 64;
 
 // SHADE: 0 VolumeShader::color over an FP32 field, 1 shaded_color (lit), 2 color over an FP64 field.
@@ -366,10 +383,10 @@ __global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) 
       if (shade)
       {
         if constexpr (LIT)
-          blend_nc (rgba, lit_color<P> (a, cell, ref, ray));
+          blend_nc (rgba, lit_color<P> (a, cell, ref, ray.dir));
         else if constexpr (SHADE == 2)
           blend_nc (rgba, color_lookup64 (a.lut, a.lut_size, a.fmin64, a.fmax64, a.inv_range64,
-                                          field_at<P, double> (a, a.field64, cell, ref)));
+                                          field_at<P> (a, a.field64, cell, ref)));
         else
           blend_nc (rgba, color_lookup (a.lut, a.lut_size, a.fmin, a.fmax, a.inv_range, field_at<P> (a, a.field, cell, ref)));
         distance += a.sample_dist;
@@ -390,7 +407,7 @@ __global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) 
   }
 }
 
-// ---- Sample-parallel form for frames with too few rays to fill the GPU at one lane per ray ----
+// ---- Sample-parallel form for frames with few rays per element ----
 // A block holds 64 rays (one per lane) and kSplitWaves wavefronts.  One round covers kSplitR consecutive
 // samples of every ray: wave w locates and shades samples [base + w*T, base + (w+1)*T) of its lane's ray
 // into LDS (a sample's location and colour depend on its point alone), then wave 0 advances each ray
@@ -413,7 +430,7 @@ __host__ __device__ constexpr int split_waves_per_simd (int P, bool polish)
 {
   return DRX_SPLIT_WAVES_PER_SIMD > 0 ? DRX_SPLIT_WAVES_PER_SIMD : waves_per_simd (P, polish, 0);
 }
-constexpr int32_t kRecFound = 1 << 30, kRecPolished = 1 << 29, kRecOverflow = 1 << 28, kRecCand = (1 << 28) - 1;
+constexpr int32_t kSplitFound = 1 << 30, kSplitPolished = 1 << 29, kSplitOverflow = 1 << 28, kSplitCand = (1 << 28) - 1;
 
 template <int P, bool POLISH, int SHADE>
 __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, POLISH)) k_integrate_split (IntegrateArgs a)
@@ -487,15 +504,15 @@ __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, PO
         float ref[3];
         const int cell = locate_point<P, POLISH> (a.cfg, todo, pt, ref, st, ovf);
         cn.x = st.newton;
-        cn.y = min (st.candidates, kRecCand) | (cell >= 0 ? kRecFound : 0) | (st.polished ? kRecPolished : 0) |
-               (ovf ? kRecOverflow : 0);
+        cn.y = min (st.candidates, kSplitCand) | (cell >= 0 ? kSplitFound : 0) | (st.polished ? kSplitPolished : 0) |
+               (ovf ? kSplitOverflow : 0);
         if (cell >= 0 && !ovf)
         {
           if constexpr (SHADE == 1)
-            col = lit_color<P> (a, cell, ref, ray);
+            col = lit_color<P> (a, cell, ref, ray.dir);
           else if constexpr (SHADE == 2)
             col = color_lookup64 (a.lut, a.lut_size, a.fmin64, a.fmax64, a.inv_range64,
-                                  field_at<P, double> (a, a.field64, cell, ref));
+                                  field_at<P> (a, a.field64, cell, ref));
           else
             col = color_lookup (a.lut, a.lut_size, a.fmin, a.fmax, a.inv_range, field_at<P> (a, a.field, cell, ref));
         }
@@ -524,15 +541,15 @@ __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, PO
         const int slot = (k - base) * 64 + lane;
         const int2 cn = rcnt[slot];
         v[1] += (unsigned)cn.x;
-        v[2] += (unsigned)(cn.y & kRecCand);
-        v[3] += (cn.y & kRecPolished) ? 1 : 0;
-        if (cn.y & kRecOverflow)
+        v[2] += (unsigned)(cn.y & kSplitCand);
+        v[3] += (cn.y & kSplitPolished) ? 1 : 0;
+        if (cn.y & kSplitOverflow)
         {
           overflow = true;
           alive = false;
           break;
         }
-        const bool found = (cn.y & kRecFound) != 0;
+        const bool found = (cn.y & kSplitFound) != 0;
         if (found) ++v[0];
         bool shade = false;
         if (!inseg)
@@ -573,6 +590,220 @@ __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, PO
         if (shade)
         {
           blend_nc (rgba, rcol[slot]);
+          distance += a.sample_dist;
+          ++k;
+        }
+      }
+      ray_live[lane] = alive;
+      const bool any = __ballot (alive) != 0;
+      if (lane == 0) more = any;
+    }
+    __syncthreads ();
+    if (!more) break;
+  }
+  if (overflow) atomicOr (a.err, 1);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+  {
+    unsigned long long x = v[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor (x, o, 64);
+    if (lane == 0 && x) atomicAdd (&a.stats[q], x);
+  }
+}
+
+// ---- Sample-parallel form with the candidates binned by element ----
+// A block holds 64 rays (one per lane) and four wavefronts.  One round covers kBinnedR consecutive samples of every
+// ray: the block locates them all at once with the candidates binned by element (locate_binned; a sample's
+// location and colour depend on its point alone), each located sample's colour goes to LDS, then wave 0 advances each
+// ray through k_integrate's march state machine over the round's samples, and the block stops when its rays
+// are done.  The sample distances come from the same float additions as the march's, and every locate the
+// march makes (including the repeated one after a segment closes) is replayed from its sample's record,
+// so partials and statistics equal k_integrate's bit for bit; samples taken past a ray's end are wasted
+// work (under kBinnedR per ray), never results.
+//
+// The vector-memory data path bounded one lane per ray (88% busy: 29 node visits and two Newton steps of 48 reads a
+// sample); here the walk is one descent per wavefront and Newton's operands are scalar, and the vector units are
+// the busier side (62%, the data path 87% with the points of small groups).  Integrate kernel against one lane per ray
+// with entry cells: 64^3 order 3, 1024^2 x 512 samples 12.4 -> 8.6 ms; 40^3 order 4, 1000^2 x 1000, FP64 polish 70 -> 50
+// ms; against the per-lane form above: 8^3 order 2, FP64 field, 256^2 x 200: 1.16 -> 0.73 ms; lit 40^3 order 3, 900^2
+// x 200: 9.6 -> 7.1 ms.  Staging the elements in LDS instead of scalar reads: 10.9 and 62 ms.
+// Waves per SIMD: four blocks fit a CU's LDS, three of the lit kernel, whose samples are colours.
+__host__ __device__ constexpr int binned_waves_per_simd (int shade) { return shade == 1 ? 3 : 4; }
+// Samples per ray and round: with 8, groups are small and rounds many (order-3 frame 16.6 ms against 14.2 ms when
+// lanes still walked by themselves; lit frames of eight 6^3 order-2 domains 3.7 ms against 2.3 ms).
+constexpr int kBinnedR = 16;
+
+template <int P, bool POLISH, int SHADE>
+__global__ void __launch_bounds__ (kBinThreads, binned_waves_per_simd (SHADE)) k_integrate_binned (IntegrateArgs a)
+{
+  constexpr int R = kBinnedR, N = 64 * R;
+  typedef std::conditional_t<SHADE == 1, float4, int32_t> Shade;
+  __shared__ BinShared<N> sh;
+  __shared__ Shade shade_rec[N];          // [sample of the round][ray]
+  __shared__ float ray_rec[7][64];        // direction, origin, distance of the round's first sample
+  __shared__ int32_t ray_live[64];
+  __shared__ int32_t more;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + lane;
+  const bool has_ray = i < a.n_rays;
+  const int ri = has_ray ? (a.order ? a.order[i] : i) : 0;
+  Ray ray;
+  if (has_ray)
+    ray = a.rays[ri];
+  else
+  {
+    ray.dir[0] = ray.dir[1] = ray.dir[2] = 0.f;
+    ray.orig[0] = ray.orig[1] = ray.orig[2] = 0.f;
+    ray.near_ = ray.far_ = 0.f;
+    ray.pixel_id = -1;
+  }
+  Partial *out5 = a.slots + 5 * (int64_t)ri;
+  if (wv == 0 && has_ray)
+#pragma unroll
+    for (int s = 0; s < 5; ++s)
+    {
+      Partial p0;
+      p0.pixel_id = -1;
+      p0.depth = INFINITY;
+      p0.rgba[0] = p0.rgba[1] = p0.rgba[2] = p0.rgba[3] = 0.f;
+      out5[s] = p0;
+    }
+  if (wv == 0)
+  {
+    ray_live[lane] = has_ray;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+      ray_rec[d][lane] = ray.dir[d];
+      ray_rec[3 + d][lane] = ray.orig[d];
+    }
+  }
+  // march state (wave 0): the distance of sample k
+  float distance = ray.near_ + a.sample_dist;
+  int k = 0, segment = 0;
+  bool inseg = false, alive = has_ray, overflow = false;
+  float depth = 0.f;
+  float rgba[4] = { 0.f, 0.f, 0.f, 0.f };
+  unsigned long long v[4] = { 0, 0, 0, 0 };   // located, Newton steps, candidates, polished
+  // the distance of this wavefront's first sample of the round and of the sample before it (the march only locates
+  // sample k when sample k - 1 lies before `far`)
+  constexpr int Q = R / kBinWaves;
+  float sd = ray.near_ + a.sample_dist, sprev = -INFINITY;
+  for (int q = 0; q < wv * Q; ++q)
+  {
+    sprev = sd;
+    sd += a.sample_dist;
+  }
+  int span = Q / 2;
+  for (int base = 0;; base += R)
+  {
+    if (wv == 0) ray_rec[6][lane] = sd;
+    __syncthreads ();   // ray_rec, ray_live
+    const bool live = ray_live[lane] != 0;
+    locate_binned<P, POLISH, N> (
+        a.cfg, sh, span,
+        [&] (int q, float pt[3]) {
+          float d = sd, prev = sprev;
+          for (int t = 0; t < q; ++t)
+          {
+            prev = d;
+            d += a.sample_dist;
+          }
+#pragma unroll
+          for (int c = 0; c < 3; ++c) pt[c] = ray_point (ray.orig[c], d, ray.dir[c]);
+          return live && prev < ray.far_;
+        },
+        [&] (int item, float pt[3]) {
+          const int j = item & 63;
+          float d = ray_rec[6][j];
+          for (int t = 0; t < (item >> 6); ++t) d += a.sample_dist;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) pt[c] = ray_point (ray_rec[3 + c][j], d, ray_rec[c][j]);
+        },
+        [&] (int item, int el, const float ref[3], auto uni) {
+          constexpr bool UNI = decltype (uni)::value;
+          if constexpr (SHADE == 1)
+          {
+            const int j = item & 63;
+            const float dir[3] = { ray_rec[0][j], ray_rec[1][j], ray_rec[2][j] };
+            shade_rec[item] = lit_color<P, UNI> (a, el, ref, dir);
+          }
+          else if constexpr (SHADE == 2)
+            shade_rec[item] = color_index64 (a.lut_size, a.fmin64, a.fmax64, a.inv_range64, field_at<P, UNI> (a, a.field64, el, ref));
+          else
+            shade_rec[item] = color_index (a.lut_size, a.fmin, a.fmax, a.inv_range, field_at<P, UNI> (a, a.field, el, ref));
+        });
+    for (int q = 0; q < R; ++q)
+    {
+      sprev = sd;
+      sd += a.sample_dist;
+    }
+    if (wv == 0)
+    {
+      while (alive)
+      {
+        if (!inseg && !(distance < ray.far_))
+        {
+          alive = false;
+          break;
+        }
+        if (k >= base + R) break;   // the next round holds this sample
+        const int slot = (k - base) * 64 + lane;
+        const uint32_t cn = sh.rec[slot];
+        v[1] += cn & kRecSteps;
+        v[2] += (cn & kRecCands) / kRecCandOne;
+        v[3] += (cn & kRecPolished) ? 1 : 0;
+        if (cn & kRecOverflow)
+        {
+          overflow = true;
+          alive = false;
+          break;
+        }
+        const bool found = (cn & kRecFound) != 0;
+        if (found) ++v[0];
+        bool shade = false;
+        if (!inseg)
+        {
+          if (found)
+          {
+            inseg = true;
+            depth = distance;
+            rgba[0] = rgba[1] = rgba[2] = rgba[3] = 0.f;
+            shade = true;
+          }
+          else
+          {
+            distance += a.sample_dist;
+            ++k;
+          }
+        }
+        else if (distance < ray.far_ && found && rgba[3] < 0.95f)
+          shade = true;
+        else
+        {
+          Partial pp;
+          pp.pixel_id = ray.pixel_id;
+          pp.depth = depth;
+          pp.rgba[0] = rgba[0];
+          pp.rgba[1] = rgba[1];
+          pp.rgba[2] = rgba[2];
+          pp.rgba[3] = rgba[3];
+          out5[segment] = pp;
+          ++segment;
+          if (distance >= ray.far_ || rgba[3] > 0.95f || segment == 5)
+          {
+            alive = false;
+            break;
+          }
+          inseg = false;
+        }
+        if (shade)
+        {
+          if constexpr (SHADE == 1)
+            blend_nc (rgba, shade_rec[slot]);
+          else
+            blend_nc (rgba, a.lut[shade_rec[slot]]);
           distance += a.sample_dist;
           ++k;
         }
@@ -700,6 +931,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   // kSplitMaxRaysPerSimd active rays per SIMD under the automatic walk and launch.
   const int launch = opts ? opts->launch : DRX_LAUNCH_AUTO;
   const bool plain = !guided && !learned && P <= DRX_MAX_MIXED_ORDER;
+  const bool binned = (double)n_rays >= kBinnedMinRaysPerColumn * std::cbrt ((double)mesh->n_el * (double)mesh->n_el);
   bool split = false;
   if (launch == DRX_LAUNCH_SAMPLES)
   {
@@ -710,9 +942,11 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   }
   else if (launch == DRX_LAUNCH_AUTO && trav == DRX_TRAVERSE_AUTO && plain)
   {
+    // large frames too where the rays are dense, but for small BVHs that carry the 8-wide copy (the wave walk)
     int dev = 0;
     split = hipGetDevice (&dev) == hipSuccess &&
-            (int64_t)n_rays < (int64_t)kSplitMaxRaysPerSimd * 4 * compute_units (dev);
+            ((int64_t)n_rays < (int64_t)kSplitMaxRaysPerSimd * 4 * compute_units (dev) ||
+             (binned && !(a.cfg.wide && bvh->n_leaves <= kWaveWalkMaxLeaves)));
   }
   int walk = split ? DRX_TRAVERSE_BINARY : trav;
   if (walk == DRX_TRAVERSE_AUTO && a.cfg.wide && !learned && P <= DRX_MAX_MIXED_ORDER)
@@ -790,7 +1024,39 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     else                                                                     \
       hipLaunchKernelGGL ((k_integrate<PP, PO, 0, 0>), g, b, 0, st, a);      \
   } while (0)
-  if (split)
+#define DRX_BINNED(PP, PO)                                                                 \
+  do                                                                                       \
+  {                                                                                        \
+    const dim3 gs (nblk (n_rays, 64)), bs (kBinThreads);                                   \
+    if (f64)                                                                               \
+      hipLaunchKernelGGL ((k_integrate_binned<PP, PO, 2>), gs, bs, 0, st, a);              \
+    else if (lit)                                                                          \
+      hipLaunchKernelGGL ((k_integrate_binned<PP, PO, 1>), gs, bs, 0, st, a);              \
+    else                                                                                   \
+      hipLaunchKernelGGL ((k_integrate_binned<PP, PO, 0>), gs, bs, 0, st, a);              \
+  } while (0)
+  if (split && binned)
+  {
+    if (a.cfg.polish)
+      switch (P)
+      {
+      case 0: DRX_BINNED (0, true); break;
+      case 1: DRX_BINNED (1, true); break;
+      case 2: DRX_BINNED (2, true); break;
+      case 3: DRX_BINNED (3, true); break;
+      default: DRX_BINNED (4, true); break;
+      }
+    else
+      switch (P)
+      {
+      case 0: DRX_BINNED (0, false); break;
+      case 1: DRX_BINNED (1, false); break;
+      case 2: DRX_BINNED (2, false); break;
+      case 3: DRX_BINNED (3, false); break;
+      default: DRX_BINNED (4, false); break;
+      }
+  }
+  else if (split)
   {
     if (a.cfg.polish)
       switch (P)
@@ -839,6 +1105,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     }
 #undef DRX_INT_HI
 #undef DRX_SPLIT
+#undef DRX_BINNED
 #undef DRX_INT
 #undef DRX_INT64
 #undef DRX_INT2

@@ -32,29 +32,35 @@ __device__ __forceinline__ void blend_nc (float f[4], const float4 b)   // rende
 
 // DeviceColorMap::color for Float = double (device_color_map.hpp:61-77): clamp and normalise in double,
 // the normalised value rounded to float32 before it is scaled to an index.
-__device__ __forceinline__ float4 color_lookup64 (const float4 *__restrict__ lut, int size, double mn, double mx,
-                                                  double inv, double scalar)
+__device__ __forceinline__ int color_index64 (int size, double mn, double mx, double inv, double scalar)
 {
 #pragma clang fp contract(off)
   const double s = fmin (mx, fmax (mn, scalar));
   const double s2 = (scalar != scalar) ? mn : s;
   const float normalized = (float)((s2 - mn) * inv);
   int idx = (int)(normalized * (float)(size - 1));
-  idx = min (max (idx, 0), size - 1);
-  return lut[idx];
+  return min (max (idx, 0), size - 1);
+}
+__device__ __forceinline__ float4 color_lookup64 (const float4 *__restrict__ lut, int size, double mn, double mx,
+                                                  double inv, double scalar)
+{
+  return lut[color_index64 (size, mn, mx, inv, scalar)];
 }
 
 // DeviceColorMap::color (device_color_map.hpp:61-77)
-__device__ __forceinline__ float4 color_lookup (const float4 *__restrict__ lut, int size, float mn, float mx, float inv,
-                                                float scalar)
+__device__ __forceinline__ int color_index (int size, float mn, float mx, float inv, float scalar)
 {
 #pragma clang fp contract(off)
   const float s = fminf (mx, fmaxf (mn, scalar));
   const float s2 = (scalar != scalar) ? mn : s;   // std::max(min, NaN) keeps min
   const float normalized = (s2 - mn) * inv;
   int idx = (int)(normalized * (float)(size - 1));
-  idx = min (max (idx, 0), size - 1);
-  return lut[idx];
+  return min (max (idx, 0), size - 1);
+}
+__device__ __forceinline__ float4 color_lookup (const float4 *__restrict__ lut, int size, float mn, float mx, float inv,
+                                                float scalar)
+{
+  return lut[color_index (size, mn, mx, inv, scalar)];
 }
 
 static inline unsigned nblk (int64_t n, int b) { return (unsigned)((n + b - 1) / b); }

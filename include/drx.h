@@ -172,8 +172,9 @@ enum drx_launch
                                  consecutive samples in parallel and one of them runs each ray's march over
                                  them (same partials and statistics; binary walk, plain start, orders up to
                                  DRX_MAX_MIXED_ORDER).  Under DRX_LAUNCH_AUTO and DRX_TRAVERSE_AUTO a render
-                                 takes it for frames of fewer than 300 active rays per SIMD; DRX_LAUNCH_CHUNKED
-                                 or DRX_LAUNCH_PERSISTENT keep one lane per ray */
+                                 takes it for frames of fewer than 300 active rays per SIMD, and for larger
+                                 ones of at least 32 active rays per element column unless the wave walk
+                                 applies; DRX_LAUNCH_CHUNKED or DRX_LAUNCH_PERSISTENT keep one lane per ray */
 };
 
 /* Training schedule of the learned initializer (drx_mlp_train): Adam, cosine decay lr -> lr_final over
@@ -204,12 +205,12 @@ typedef struct drx_integrate_stats
 {
   int64_t located_samples;    /* successful locate() calls inside the march */
   int64_t newton_steps;       /* Newton iterations over all candidates */
-  int64_t candidates;         /* candidate leaves tried */
+  int64_t candidates;         /* candidate leaves tried (sample-parallel launch: up to 4,095 counted a sample) */
   int64_t polished;           /* samples that took the FP64 correction */
   float kernel_ms;            /* duration of the integrate kernel alone (HIP events on `stream`) */
   float total_ms;             /* the whole call: integrate + partial compaction (HIP events) */
   int32_t walk;               /* the walk that ran: 0 binary, 1 8-wide per lane, 2 wave-coherent, 3 learned start,
-                                 4 binary with given starts / record, 5 binary, sample-parallel launch */
+                                 4 binary with given starts / record, 5 binary walk's candidates, sample-parallel launch */
 } drx_integrate_stats;
 
 /* PointLight (rendering/point_light.hpp:15-33); dray's defaults: amb 0.4, diff 0.75, spec 0.8, spec_pow 15. */
