@@ -88,10 +88,11 @@ static_assert (sizeof (Location) == 16, "Location layout");
 inline int npe_of (int p) { return (p + 1) * (p + 1) * (p + 1); }
 inline int npe_pad_of (int p) { return (npe_of (p) + 3) & ~3; }
 
-// Exclusive scan of int32 flags (device), n elements; writes scan[n] and *total (host).  The block sums
-// live in `sums` (scan_sums_len(n) int32) when given, else in the arena's scan slot.
+// Exclusive scan of int32 flags (device), n elements; writes scan[n] and *total (host, waits for it).  The block sums
+// live in `sums` (scan_sums_len(n) int32) when given, else in the arena's scan slot.  total_dev (device, nullable)
+// takes the total without waiting.
 int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *total_host, hipStream_t st,
-                        int32_t *sums = nullptr);
+                        int32_t *sums = nullptr, int32_t *total_dev = nullptr);
 int32_t scan_sums_len (int32_t n);
 
 // Stable LSD radix sort of (key, value) pairs over the low `bits` bits (8-bit digits); ping-pongs between

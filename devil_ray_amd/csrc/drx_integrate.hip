@@ -826,17 +826,18 @@ __global__ void __launch_bounds__ (kBinThreads, binned_waves_per_simd (SHADE)) k
   }
 }
 
-__global__ void k_flag_partials (const Partial *__restrict__ p, int64_t n, int32_t *__restrict__ flags)
+__global__ void __launch_bounds__ (kCompactThreads) k_count_partials (const Partial *__restrict__ p, int64_t n,
+                                                                       int32_t *__restrict__ counts)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) flags[i] = (p[i].depth == INFINITY) ? 0 : 1;
+  compact_count (n, counts, [&] (int64_t i) { return p[i].depth != INFINITY; });
 }
 
-__global__ void k_compact_partials (const Partial *__restrict__ p, int64_t n, const int32_t *__restrict__ flags,
-                                    const int32_t *__restrict__ pos, Partial *__restrict__ out)
+__global__ void __launch_bounds__ (kCompactThreads) k_compact_partials (const Partial *__restrict__ p, int64_t n,
+                                                                         const int32_t *__restrict__ counts, bool scanned,
+                                                                         int32_t *__restrict__ total,
+                                                                         Partial *__restrict__ out)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && flags[i]) out[pos[i]] = p[i];
+  compact_put (n, counts, scanned, total, [&] (int64_t i) { return p[i].depth != INFINITY; }, [&] (int64_t i, int32_t k) { out[k] = p[i]; });
 }
 
 } // namespace drx
@@ -886,10 +887,11 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   hipStream_t st = as_stream (stream);
   const int64_t n_slots = 5 * (int64_t)n_rays;
   Partial *slots = (Partial *)arena (SLOT_PARTIALS, sizeof (Partial) * (size_t)n_slots, st);
-  int32_t *flags = (int32_t *)arena (SLOT_FLAGS, sizeof (int32_t) * 2 * (size_t)n_slots + 64, st);
+  const int32_t n_blocks = compact_blocks (n_slots);
+  int32_t *counts = (int32_t *)arena (SLOT_FLAGS, sizeof (int32_t) * 2 * (size_t)n_blocks + 64, st);
   unsigned long long *dstats = (unsigned long long *)arena (SLOT_STATS, 8 * sizeof (unsigned long long), st);
-  if (!slots || !flags || !dstats) return DRX_ERR_HIP;
-  int32_t *pos = flags + n_slots;
+  if (!slots || !counts || !dstats) return DRX_ERR_HIP;
+  int32_t *first = counts + n_blocks;
   int32_t *err = (int32_t *)(dstats + 4);
   hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)16, 0);
   IntegrateArgs a;
@@ -1112,18 +1114,18 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   DRX_LAUNCH_CHECK ();
   DRX_HIP (hipEventRecord (ev[1], st));
   DRX_LAUNCH_CHECK ();
-  hipLaunchKernelGGL (k_flag_partials, dim3 (nblk (n_slots, 256)), dim3 (256), 0, st, slots, n_slots, flags);
+  hipLaunchKernelGGL (k_count_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots, counts);
   DRX_LAUNCH_CHECK ();
-  int32_t total = 0;
-  rc = exclusive_scan_i32 (flags, pos, (int32_t)n_slots, &total, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL (k_compact_partials, dim3 (nblk (n_slots, 256)), dim3 (256), 0, st, slots, n_slots, flags, pos,
-                      (Partial *)out_partials);
+  const bool scanned = n_blocks > kCompactSelfScan;
+  if (scanned && (rc = exclusive_scan_i32 (counts, first, n_blocks, nullptr, st))) return rc;
+  hipLaunchKernelGGL (k_compact_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots,
+                      scanned ? first : counts, scanned, err + 1, (Partial *)out_partials);
   DRX_LAUNCH_CHECK ();
   DRX_HIP (hipEventRecord (ev[2], st));
   unsigned long long hs[8];
   DRX_HIP (hipMemcpyAsync (hs, dstats, sizeof hs, hipMemcpyDeviceToHost, st));
   DRX_HIP (hipStreamSynchronize (st));
+  const int32_t total = ((int32_t *)(hs + 4))[1];
   float k_ms = 0.f, t_ms = 0.f;
   DRX_HIP (hipEventElapsedTime (&k_ms, ev[0], ev[1]));
   DRX_HIP (hipEventElapsedTime (&t_ms, ev[0], ev[2]));

@@ -570,25 +570,30 @@ __device__ __forceinline__ bool ray_slab (const Ray &ray, const Bounds6 &mb, flo
   return maxd > mind;
 }
 
-__global__ void k_mark_active (const Ray *__restrict__ rays, int n, Bounds6 mb, int32_t *__restrict__ flags)
+__global__ void __launch_bounds__ (kCompactThreads) k_count_active (const Ray *__restrict__ rays, int n, Bounds6 mb,
+                                                                     int32_t *__restrict__ counts)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float a, b;
-  flags[i] = ray_slab (rays[i], mb, a, b) ? 1 : 0;
+  compact_count (n, counts, [&] (int64_t i) {
+    float a, b;
+    return ray_slab (rays[i], mb, a, b);
+  });
 }
 
-__global__ void k_gather_active (const Ray *__restrict__ rays, int n, Bounds6 mb, const int32_t *__restrict__ flags,
-                                 const int32_t *__restrict__ pos, Ray *__restrict__ out)
+__global__ void __launch_bounds__ (kCompactThreads) k_gather_active (const Ray *__restrict__ rays, int n, Bounds6 mb,
+                                                                      const int32_t *__restrict__ counts, bool scanned,
+                                                                      int32_t *__restrict__ total, Ray *__restrict__ out)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || !flags[i]) return;
-  Ray r = rays[i];
-  float nr, fr;
-  ray_slab (r, mb, nr, fr);
-  r.near_ = nr;
-  r.far_ = fr;
-  out[pos[i]] = r;
+  compact_put (
+      n, counts, scanned, total,
+      [&] (int64_t i) {
+        float a, b;
+        return ray_slab (rays[i], mb, a, b);
+      },
+      [&] (int64_t i, int32_t k) {
+        Ray r = rays[i];
+        ray_slab (r, mb, r.near_, r.far_);
+        out[k] = r;
+      });
 }
 
 // Ray tiles of 64 pixels, kTileW x kTileH (one wavefront each).
@@ -616,40 +621,151 @@ __global__ void k_tile_scatter (const Ray *__restrict__ rays, int n, int w, int 
 }
 
 // Tile keys for longest-first processing: the longest [near, far] segment among the tile's rays, as a
-// descending unsigned key (tiles without rays sort last).
-__global__ void k_tile_keys (const Ray *__restrict__ rays, const int32_t *__restrict__ slots, int n_tiles,
-                             uint32_t *__restrict__ keys, int32_t *__restrict__ vals)
+// descending unsigned key (tiles without rays sort last), and the tile's ray count.  One wavefront per tile.
+__global__ void __launch_bounds__ (256) k_tile_keys (const Ray *__restrict__ rays, const int32_t *__restrict__ slots,
+                                                     int n_tiles, uint32_t *__restrict__ keys, int32_t *__restrict__ vals,
+                                                     int32_t *__restrict__ counts)
 {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= n_tiles) return;
+  const int r = slots[((int64_t)t << 6) + lane];
   float len = -1.f;
-  for (int l = 0; l < 64; ++l)
+  if (r >= 0) len = fmaxf (len, fmaxf (rays[r].far_ - rays[r].near_, 0.f));
+  len = wave_reduce_max (len);
+  const int c = __popcll (__ballot (r >= 0));
+  if (lane == 0)
   {
-    const int r = slots[((int64_t)t << 6) + l];
-    if (r >= 0) len = fmaxf (len, fmaxf (rays[r].far_ - rays[r].near_, 0.f));
+    keys[t] = len < 0.f ? 0xFFFFFFFFu : 0x7FFFFFFFu - __float_as_uint (len);
+    vals[t] = t;
+    counts[t] = c;
   }
-  keys[t] = len < 0.f ? 0xFFFFFFFFu : 0x7FFFFFFFu - __float_as_uint (len);
-  vals[t] = t;
 }
 
-__global__ void k_gather_tiles (const int32_t *__restrict__ slots, const int32_t *__restrict__ perm, int64_t n,
-                                int32_t *__restrict__ out)
+__global__ void k_gather_i32 (const int32_t *__restrict__ v, const int32_t *__restrict__ perm, int n, int32_t *__restrict__ out)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = slots[((int64_t)perm[i >> 6] << 6) + (i & 63)];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = v[perm[i]];
 }
 
-__global__ void k_flag_nonneg (const int32_t *__restrict__ v, int64_t n, int32_t *__restrict__ flags)
+// The processing order: the rays of the tiles in sorted order, each tile's from its first place on.
+__global__ void __launch_bounds__ (256) k_tile_order (const int32_t *__restrict__ slots, const int32_t *__restrict__ perm,
+                                                      const int32_t *__restrict__ first, int n_tiles,
+                                                      int32_t *__restrict__ out)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) flags[i] = v[i] >= 0 ? 1 : 0;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= n_tiles) return;
+  const int r = slots[((int64_t)perm[i] << 6) + lane];
+  const uint64_t b = __ballot (r >= 0);
+  if (r >= 0) out[first[i] + __popcll (b & ((1ull << lane) - 1))] = r;
 }
 
-__global__ void k_compact_i32 (const int32_t *__restrict__ v, int64_t n, const int32_t *__restrict__ pos,
-                               int32_t *__restrict__ out)
+// Stable sort of up to kSmallSort (key, value = index) pairs and the exclusive scan of counts[] in sorted order, by one
+// block: the LDS holds the pairs between the passes, wavefront w owns the w-th run of them and ranks it like
+// k_radix_scatter.  For the few thousand tiles of a frame the passes' launches cost more than their work: a
+// chain of four passes in one block (4,096 tiles: 25 us) against 12 launches of 5.6 to 7.5 us and the gaps between
+// them.  Latency-bound; up to kSmallSort tiles (what the LDS holds, a 1,024^2 frame), beyond it the launched passes.
+constexpr int kSmallSortThreads = 1024, kSmallSortRounds = 16, kSmallSort = kSmallSortThreads * kSmallSortRounds;
+
+__global__ void __launch_bounds__ (kSmallSortThreads) k_sort_small (const uint32_t *__restrict__ keys, const int32_t *__restrict__ counts,
+                                                                     int n, int32_t *__restrict__ perm,
+                                                                     int32_t *__restrict__ first, int32_t *__restrict__ total)
 {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && v[i] >= 0) out[pos[i]] = v[i];
+  constexpr int W = kSmallSortThreads / 64;
+  __shared__ uint32_t lk[kSmallSort];
+  __shared__ uint16_t lv[kSmallSort];
+  __shared__ int32_t at[W][256];
+  __shared__ int32_t wsum[W];
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const uint64_t lt = lanemask_lt ();
+  const int rounds = (n + kSmallSortThreads - 1) / kSmallSortThreads, base = w * (rounds * 64) + lane;
+  for (int i = tid; i < n; i += kSmallSortThreads)
+  {
+    lk[i] = keys[i];
+    lv[i] = (uint16_t)i;
+  }
+  for (int shift = 0; shift < 32; shift += 8)
+  {
+    for (int q = tid; q < W * 256; q += kSmallSortThreads) (&at[0][0])[q] = 0;
+    __syncthreads ();
+    uint32_t key[kSmallSortRounds];
+    int32_t val[kSmallSortRounds], rank[kSmallSortRounds]; // rank among the wavefront's equal digits
+#pragma unroll
+    for (int r = 0; r < kSmallSortRounds; ++r)
+      if (r < rounds)
+      {
+        const int i = base + 64 * r;
+        const bool valid = i < n;
+        key[r] = valid ? lk[i] : 0u;
+        val[r] = valid ? lv[i] : 0;
+        const uint32_t digit = (key[r] >> shift) & 0xFF;
+        uint64_t peers = __ballot (valid);
+        if (!valid) peers = ~peers;
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+        {
+          const uint64_t m = __ballot ((digit >> b) & 1u);
+          peers &= ((digit >> b) & 1u) ? m : ~m;
+        }
+        const int before = at[w][digit];
+        __builtin_amdgcn_fence (__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier ();
+        rank[r] = before + __popcll (peers & lt);
+        if (valid && (peers & lt) == 0) at[w][digit] = before + __popcll (peers);
+        __builtin_amdgcn_fence (__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_wave_barrier ();
+      }
+    __syncthreads ();
+    // digit totals -> first places (threads 0..255), then each wavefront's share
+    int32_t s = 0;
+    if (tid < 256)
+      for (int q = 0; q < W; ++q)
+      {
+        const int32_t c = at[q][tid];
+        at[q][tid] = s;
+        s += c;
+      }
+    const int32_t incl = wave_scan_incl_add (s);
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads ();
+    if (tid < 256)
+    {
+      int32_t o = incl - s;
+      for (int q = 0; q < w; ++q) o += wsum[q];
+      for (int q = 0; q < W; ++q) at[q][tid] += o;
+    }
+    __syncthreads ();
+#pragma unroll
+    for (int r = 0; r < kSmallSortRounds; ++r)
+      if (r < rounds && base + 64 * r < n)
+      {
+        const int32_t to = at[w][(key[r] >> shift) & 0xFF] + rank[r];
+        lk[to] = key[r];
+        lv[to] = (uint16_t)val[r];
+      }
+    __syncthreads ();
+  }
+  int32_t carry = 0;
+  for (int i0 = 0; i0 < n; i0 += kSmallSortThreads)
+  {
+    const int i = i0 + tid, t = i < n ? lv[i] : 0;
+    const int32_t c = i < n ? counts[t] : 0;
+    const int32_t incl = wave_scan_incl_add (c);
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads ();
+    int32_t o = carry + incl - c;
+    for (int q = 0; q < W; ++q)
+    {
+      o += q < w ? wsum[q] : 0;
+      carry += wsum[q];
+    }
+    if (i < n)
+    {
+      perm[i] = t;
+      first[i] = o;
+    }
+    __syncthreads ();
+  }
+  if (tid == 0) *total = carry;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1235,17 +1351,20 @@ int drx_remove_missed_rays (const void *rays, int32_t n, const float *bounds6, v
     mb.b[2 * d + 1] = hi;
   }
   hipStream_t st = as_stream (stream);
-  int32_t *flags = (int32_t *)arena (SLOT_FLAGS, sizeof (int32_t) * 2 * (size_t)n + 64, st);
-  if (!flags) return DRX_ERR_HIP;
-  int32_t *pos = flags + n;
-  hipLaunchKernelGGL (k_mark_active, dim3 (nblk (n, 256)), dim3 (256), 0, st, (const Ray *)rays, n, mb, flags);
+  const int32_t n_blocks = compact_blocks (n);
+  int32_t *counts = (int32_t *)arena (SLOT_FLAGS, sizeof (int32_t) * (2 * (size_t)n_blocks + 1) + 64, st);
+  if (!counts) return DRX_ERR_HIP;
+  int32_t *first = counts + n_blocks, *dtotal = first + n_blocks;
+  hipLaunchKernelGGL (k_count_active, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, (const Ray *)rays, n, mb, counts);
+  DRX_LAUNCH_CHECK ();
+  const bool scanned = n_blocks > kCompactSelfScan;
+  if (scanned)
+    if (int rc = exclusive_scan_i32 (counts, first, n_blocks, nullptr, st)) return rc;
+  hipLaunchKernelGGL (k_gather_active, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, (const Ray *)rays, n, mb,
+                      scanned ? first : counts, scanned, dtotal, (Ray *)out_rays);
   DRX_LAUNCH_CHECK ();
   int32_t total = 0;
-  int rc = exclusive_scan_i32 (flags, pos, n, &total, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL (k_gather_active, dim3 (nblk (n, 256)), dim3 (256), 0, st, (const Ray *)rays, n, mb, flags, pos,
-                      (Ray *)out_rays);
-  DRX_LAUNCH_CHECK ();
+  DRX_HIP (hipMemcpyAsync (&total, dtotal, sizeof total, hipMemcpyDeviceToHost, st));
   DRX_HIP (hipStreamSynchronize (st));
   *out_count = total;
   return DRX_OK;
@@ -1260,39 +1379,43 @@ int drx_ray_tile_order (const void *rays, int32_t n, int32_t width, int32_t heig
   const int tiles_x = (width + kTileW - 1) / kTileW, tiles_y = (height + kTileH - 1) / kTileH;
   const int64_t slots_n = (int64_t)tiles_x * tiles_y * 64;
   if (slots_n > (1ll << 30)) return fail (DRX_ERR_ARG, "drx_ray_tile_order: image too large");
-  int32_t *slots0 = (int32_t *)arena (SLOT_TREE2, sizeof (int32_t) * 4 * (size_t)slots_n + 64, st);
-  if (!slots0) return DRX_ERR_HIP;
-  int32_t *slots = slots0 + slots_n, *flags = slots + slots_n, *pos = flags + slots_n;
-  hipLaunchKernelGGL (k_fill_i32q, dim3 (nblk (slots_n, 256)), dim3 (256), 0, st, slots0, slots_n, -1);
-  hipLaunchKernelGGL (k_tile_scatter, dim3 (nblk (n, 256)), dim3 (256), 0, st, (const Ray *)rays, n, width, height, slots0);
+  const int n_img_tiles = tiles_x * tiles_y;
+  int32_t *slots = (int32_t *)arena (SLOT_TREE2, sizeof (int32_t) * ((size_t)slots_n + 4 * (size_t)n_img_tiles + 1) + 64, st);
+  uint32_t *kA = (uint32_t *)arena (SLOT_SORT_KEYS_A, sizeof (uint32_t) * (size_t)n_img_tiles, st);
+  int32_t *vA = (int32_t *)arena (SLOT_SORT_VALS_A, sizeof (int32_t) * (size_t)n_img_tiles, st);
+  if (!slots || !kA || !vA) return DRX_ERR_HIP;
+  int32_t *counts = slots + slots_n, *perm = counts + n_img_tiles, *sorted = perm + n_img_tiles, *first = sorted + n_img_tiles,
+          *dtotal = first + n_img_tiles;
+  hipLaunchKernelGGL (k_fill_i32q, dim3 (nblk (slots_n, 256)), dim3 (256), 0, st, slots, slots_n, -1);
+  hipLaunchKernelGGL (k_tile_scatter, dim3 (nblk (n, 256)), dim3 (256), 0, st, (const Ray *)rays, n, width, height, slots);
   DRX_LAUNCH_CHECK ();
   // Tiles longest-first (stable): a frame needs more wavefronts than the GPU holds at once, and the ones
   // dispatched last run on an emptying GPU, so they should be the short ones.
-  const int n_img_tiles = tiles_x * tiles_y;
-  const int n_rt = radix_tiles (n_img_tiles);
-  uint32_t *kA = (uint32_t *)arena (SLOT_SORT_KEYS_A, sizeof (uint32_t) * (size_t)n_img_tiles, st);
-  uint32_t *kB = (uint32_t *)arena (SLOT_SORT_KEYS_B, sizeof (uint32_t) * (size_t)n_img_tiles, st);
-  int32_t *vA = (int32_t *)arena (SLOT_SORT_VALS_A, sizeof (int32_t) * (size_t)n_img_tiles, st);
-  int32_t *vB = (int32_t *)arena (SLOT_SORT_VALS_B, sizeof (int32_t) * (size_t)n_img_tiles, st);
-  int32_t *hist = (int32_t *)arena (SLOT_SORT_HIST, sizeof (int32_t) * (2 * 256 * (size_t)n_rt + 8), st);
-  if (!kA || !kB || !vA || !vB || !hist) return DRX_ERR_HIP;
-  hipLaunchKernelGGL (k_tile_keys, dim3 (nblk (n_img_tiles, 256)), dim3 (256), 0, st, (const Ray *)rays, slots0,
-                      n_img_tiles, kA, vA);
+  hipLaunchKernelGGL (k_tile_keys, dim3 (nblk (n_img_tiles, 4)), dim3 (256), 0, st, (const Ray *)rays, slots, n_img_tiles, kA,
+                      vA, counts);
   DRX_LAUNCH_CHECK ();
-  uint32_t *ks;
-  int32_t *vs;
-  int rc0 = radix_sort_pairs (kA, vA, kB, vB, hist, n_img_tiles, 32, st, &ks, &vs);
-  if (rc0) return rc0;
-  hipLaunchKernelGGL (k_gather_tiles, dim3 (nblk (slots_n, 256)), dim3 (256), 0, st, slots0, vs, slots_n, slots);
-  hipLaunchKernelGGL (k_flag_nonneg, dim3 (nblk (slots_n, 256)), dim3 (256), 0, st, slots, slots_n, flags);
+  if (n_img_tiles <= kSmallSort)
+    hipLaunchKernelGGL (k_sort_small, dim3 (1), dim3 (kSmallSortThreads), 0, st, kA, counts, n_img_tiles, perm, first, dtotal);
+  else
+  {
+    const int n_rt = radix_tiles (n_img_tiles);
+    uint32_t *kB = (uint32_t *)arena (SLOT_SORT_KEYS_B, sizeof (uint32_t) * (size_t)n_img_tiles, st);
+    int32_t *vB = (int32_t *)arena (SLOT_SORT_VALS_B, sizeof (int32_t) * (size_t)n_img_tiles, st);
+    int32_t *hist = (int32_t *)arena (SLOT_SORT_HIST, sizeof (int32_t) * (2 * 256 * (size_t)n_rt + 8), st);
+    if (!kB || !vB || !hist) return DRX_ERR_HIP;
+    uint32_t *ks;
+    int rc = radix_sort_pairs (kA, vA, kB, vB, hist, n_img_tiles, 32, st, &ks, &perm);
+    if (rc) return rc;
+    hipLaunchKernelGGL (k_gather_i32, dim3 (nblk (n_img_tiles, 256)), dim3 (256), 0, st, counts, perm, n_img_tiles, sorted);
+    if ((rc = exclusive_scan_i32 (sorted, first, n_img_tiles, nullptr, st, nullptr, dtotal))) return rc;
+  }
+  hipLaunchKernelGGL (k_tile_order, dim3 (nblk (n_img_tiles, 4)), dim3 (256), 0, st, slots, perm, first, n_img_tiles, out_order);
   DRX_LAUNCH_CHECK ();
   int32_t total = 0;
-  int rc = exclusive_scan_i32 (flags, pos, (int32_t)slots_n, &total, st);
-  if (rc) return rc;
+  DRX_HIP (hipMemcpyAsync (&total, dtotal, sizeof total, hipMemcpyDeviceToHost, st));
+  DRX_HIP (hipStreamSynchronize (st));
   if (total != n)
     return fail (DRX_ERR_ARG, "drx_ray_tile_order: rays are not distinct pixels of a %dx%d image", width, height);
-  hipLaunchKernelGGL (k_compact_i32, dim3 (nblk (slots_n, 256)), dim3 (256), 0, st, slots, slots_n, pos, out_order);
-  DRX_LAUNCH_CHECK ();
   return DRX_OK;
 }
 

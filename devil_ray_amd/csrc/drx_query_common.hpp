@@ -3,6 +3,7 @@
 
 #include "drx_common.hpp"
 #include "drx_element.hpp"
+#include "drx_wave.hpp"
 
 namespace drx
 {
@@ -110,6 +111,65 @@ static __global__ void k_fill_i32q (int32_t *p, int64_t n, int32_t v)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
+}
+
+// Order-preserving compaction in two passes over the items (keep (i): whether item i stays; put (i, k): writes it as
+// the k-th kept one): kept items per block, then their places.  A block takes kCompactBlock items, each wavefront a
+// quarter of them in a row.  One flag and one scan entry per item took two launches more and, for the 1.3 M partial
+// slots of a 512^2 frame, 16 MB of traffic.  Up to kCompactSelfScan blocks (4 M items) each block of the second pass
+// adds up the counts before its own, 16 loads per thread at most, which costs less than the launch of a scan (5 us and
+// the gap); with more the counts are scanned first.
+constexpr int kCompactThreads = 256, kCompactRounds = 4, kCompactBlock = kCompactThreads * kCompactRounds;
+constexpr int kCompactSelfScan = 4096;
+inline int32_t compact_blocks (int64_t n) { return (int32_t)((n + kCompactBlock - 1) / kCompactBlock); }
+
+template <typename Keep> __device__ __forceinline__ void compact_count (int64_t n, int32_t *counts, Keep &&keep)
+{
+  __shared__ int32_t wcnt[kCompactThreads / 64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t i0 = (int64_t)blockIdx.x * kCompactBlock + w * (64 * kCompactRounds) + lane;
+  int32_t c = 0;
+#pragma unroll
+  for (int r = 0; r < kCompactRounds; ++r) c += __popcll (__ballot (i0 + 64 * r < n && keep (i0 + 64 * r)));
+  if (lane == 0) wcnt[w] = c;
+  __syncthreads ();
+  if (threadIdx.x == 0) counts[blockIdx.x] = (wcnt[0] + wcnt[1]) + (wcnt[2] + wcnt[3]);
+}
+
+template <typename Keep, typename Put>
+__device__ __forceinline__ void compact_put (int64_t n, const int32_t *counts, bool scanned, int32_t *total, Keep &&keep,
+                                             Put &&put)
+{
+  __shared__ int32_t wcnt[kCompactThreads / 64], wbefore[kCompactThreads / 64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t i0 = (int64_t)blockIdx.x * kCompactBlock + w * (64 * kCompactRounds) + lane;
+  uint64_t b[kCompactRounds];
+  int32_t c = 0;
+#pragma unroll
+  for (int r = 0; r < kCompactRounds; ++r)
+  {
+    b[r] = __ballot (i0 + 64 * r < n && keep (i0 + 64 * r));
+    c += __popcll (b[r]);
+  }
+  int32_t before = 0;
+  if (!scanned)
+    for (int q = threadIdx.x; q < (int)blockIdx.x; q += kCompactThreads) before += counts[q];
+  before = wave_scan_incl_add (before);
+  if (lane == 63)
+  {
+    wcnt[w] = c;
+    wbefore[w] = before;
+  }
+  __syncthreads ();
+  int32_t k = scanned ? counts[blockIdx.x] : (wbefore[0] + wbefore[1]) + (wbefore[2] + wbefore[3]);
+  if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *total = k + (wcnt[0] + wcnt[1]) + (wcnt[2] + wcnt[3]);
+  for (int q = 0; q < w; ++q) k += wcnt[q];
+#pragma unroll
+  for (int r = 0; r < kCompactRounds; ++r)
+  {
+    if ((b[r] >> lane) & 1ull) put (i0 + 64 * r, k + __popcll (b[r] & ((1ull << lane) - 1)));
+    k += __popcll (b[r]);
+  }
 }
 
 static inline int check_mesh (const drx_mesh *m, int ncomp, const char *what)

@@ -158,7 +158,7 @@ __global__ void __launch_bounds__ (kScanBlock) k_scan_reduce (const int32_t *in,
 }
 
 // Single block: exclusive scan of block_sums in place; total -> block_sums[nb].
-__global__ void __launch_bounds__ (kScanBlock) k_scan_sums (int32_t *block_sums, int32_t nb)
+__global__ void __launch_bounds__ (kScanBlock) k_scan_sums (int32_t *block_sums, int32_t nb, int32_t *total)
 {
   __shared__ int32_t wsum[kScanBlock / 64];
   __shared__ int32_t carry;
@@ -180,6 +180,7 @@ __global__ void __launch_bounds__ (kScanBlock) k_scan_sums (int32_t *block_sums,
     __syncthreads ();
   }
   if (threadIdx.x == 0) block_sums[nb] = carry;
+  if (threadIdx.x == 0 && total) *total = carry;
 }
 
 __global__ void __launch_bounds__ (kScanBlock) k_scan_down (const int32_t *in, int32_t *out, int32_t n,
@@ -208,10 +209,11 @@ __global__ void __launch_bounds__ (kScanBlock) k_scan_down (const int32_t *in, i
 }
 
 // Small arrays (the digit counts of a sort of up to half a million keys, the flags of small frames): one block walks the
-// array with a carry, one launch instead of three (8,704 counts: 10 us against 12 us and two launches).  total -> *total.
+// array with a carry, one launch instead of three (8,704 counts: 10 us against 12 us and two launches).
 constexpr int kScanSmallBlock = 1024, kScanSmallItems = 8, kScanSmallMax = 4 * kScanSmallBlock * kScanSmallItems;
 
-__global__ void __launch_bounds__ (kScanSmallBlock) k_scan_small (const int32_t *in, int32_t *out, int32_t n, int32_t *total)
+__global__ void __launch_bounds__ (kScanSmallBlock) k_scan_small (const int32_t *in, int32_t *out, int32_t n, int32_t *sum,
+                                                                   int32_t *total)
 {
   __shared__ int32_t wsum[kScanSmallBlock / 64];
   const int w = threadIdx.x >> 6;
@@ -246,12 +248,14 @@ __global__ void __launch_bounds__ (kScanSmallBlock) k_scan_small (const int32_t 
     }
     __syncthreads ();
   }
-  if (threadIdx.x == 0) *total = carry;
+  if (threadIdx.x == 0) *sum = carry;
+  if (threadIdx.x == 0 && total) *total = carry;
 }
 
 int32_t scan_sums_len (int32_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
-int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *total_host, hipStream_t st, int32_t *sums)
+int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *total_host, hipStream_t st, int32_t *sums,
+                        int32_t *total_dev)
 {
   if (n <= 0)
   {
@@ -262,11 +266,11 @@ int exclusive_scan_i32 (const int32_t *in, int32_t *out, int32_t n, int32_t *tot
   if (!sums) sums = (int32_t *)arena (SLOT_SCAN, sizeof (int32_t) * (nb + 1), st);
   if (!sums) return DRX_ERR_HIP;
   if (n <= kScanSmallMax)
-    hipLaunchKernelGGL (k_scan_small, dim3 (1), dim3 (kScanSmallBlock), 0, st, in, out, n, sums + nb);
+    hipLaunchKernelGGL (k_scan_small, dim3 (1), dim3 (kScanSmallBlock), 0, st, in, out, n, sums + nb, total_dev);
   else
   {
     hipLaunchKernelGGL (k_scan_reduce, dim3 (nb), dim3 (kScanBlock), 0, st, in, n, sums);
-    hipLaunchKernelGGL (k_scan_sums, dim3 (1), dim3 (kScanBlock), 0, st, sums, nb);
+    hipLaunchKernelGGL (k_scan_sums, dim3 (1), dim3 (kScanBlock), 0, st, sums, nb, total_dev);
     hipLaunchKernelGGL (k_scan_down, dim3 (nb), dim3 (kScanBlock), 0, st, in, out, n, sums);
   }
   DRX_LAUNCH_CHECK ();
