@@ -55,6 +55,8 @@ enum ArenaSlot
   SLOT_COUNT
 };
 void *arena (int slot, size_t bytes, hipStream_t stream);   // nullptr + error set on failure
+// Copies a few bytes from the device to the host, in stream order, and waits for them.
+int read_back (void *host, const void *device, size_t bytes, hipStream_t stream);
 int arena_release ();
 
 inline hipStream_t as_stream (void *s) { return reinterpret_cast<hipStream_t> (s); }

@@ -1123,8 +1123,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   DRX_LAUNCH_CHECK ();
   DRX_HIP (hipEventRecord (ev[2], st));
   unsigned long long hs[8];
-  DRX_HIP (hipMemcpyAsync (hs, dstats, sizeof hs, hipMemcpyDeviceToHost, st));
-  DRX_HIP (hipStreamSynchronize (st));
+  if ((rc = read_back (hs, dstats, sizeof hs, st))) return rc;
   const int32_t total = ((int32_t *)(hs + 4))[1];
   float k_ms = 0.f, t_ms = 0.f;
   DRX_HIP (hipEventElapsedTime (&k_ms, ev[0], ev[1]));

@@ -1189,9 +1189,7 @@ int drx_bvh_build (const float *aabbs_in, const int32_t *prims_in, int32_t n_in,
   hipLaunchKernelGGL (k_emit, dim3 (nblk (inner, 256)), dim3 (256), 0, st, left, right, s_aabbs, i_aabbs, inner,
                       (float4 *)out_inner);
   DRX_LAUNCH_CHECK ();
-  DRX_HIP (hipMemcpyAsync (out_bounds, dbounds, 6 * sizeof (float), hipMemcpyDeviceToHost, st));
-  DRX_HIP (hipStreamSynchronize (st));
-  return DRX_OK;
+  return read_back (out_bounds, dbounds, 6 * sizeof (float), st);
 }
 
 int drx_bvh_pack_leaves (const drx_bvh *bvh, float *out_leaf_pack, void *stream)

@@ -1149,8 +1149,15 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
 #undef DRX_LOC_HI
   DRX_LAUNCH_CHECK ();
   int32_t herr = 0;
-  DRX_HIP (hipMemcpyAsync (&herr, err, sizeof (int32_t), hipMemcpyDeviceToHost, st));
-  DRX_HIP (hipStreamSynchronize (st));
+  if (!counters)
+  {
+    if (int rc = read_back (&herr, err, sizeof (int32_t), st)) return rc;
+  }
+  else   // drx_locate_noalloc: no pinned block is made for the stream
+  {
+    DRX_HIP (hipMemcpyAsync (&herr, err, sizeof (int32_t), hipMemcpyDeviceToHost, st));
+    DRX_HIP (hipStreamSynchronize (st));
+  }
   if (herr) return fail (DRX_ERR_OVERFLOW, "drx_locate: BVH traversal stack (%d entries) overflowed", kStackDepth);
   return DRX_OK;
 }
@@ -1364,8 +1371,7 @@ int drx_remove_missed_rays (const void *rays, int32_t n, const float *bounds6, v
                       scanned ? first : counts, scanned, dtotal, (Ray *)out_rays);
   DRX_LAUNCH_CHECK ();
   int32_t total = 0;
-  DRX_HIP (hipMemcpyAsync (&total, dtotal, sizeof total, hipMemcpyDeviceToHost, st));
-  DRX_HIP (hipStreamSynchronize (st));
+  if (int rc = read_back (&total, dtotal, sizeof total, st)) return rc;
   *out_count = total;
   return DRX_OK;
 }
@@ -1412,8 +1418,7 @@ int drx_ray_tile_order (const void *rays, int32_t n, int32_t width, int32_t heig
   hipLaunchKernelGGL (k_tile_order, dim3 (nblk (n_img_tiles, 4)), dim3 (256), 0, st, slots, perm, first, n_img_tiles, out_order);
   DRX_LAUNCH_CHECK ();
   int32_t total = 0;
-  DRX_HIP (hipMemcpyAsync (&total, dtotal, sizeof total, hipMemcpyDeviceToHost, st));
-  DRX_HIP (hipStreamSynchronize (st));
+  if (int rc = read_back (&total, dtotal, sizeof total, st)) return rc;
   if (total != n)
     return fail (DRX_ERR_ARG, "drx_ray_tile_order: rays are not distinct pixels of a %dx%d image", width, height);
   return DRX_OK;
