@@ -239,7 +239,7 @@ class LocateOptions:
     fp64_polish: bool = False
     cond_threshold: float = 1e4
     traversal: int = 0          # 0 auto (= 3), 1 per lane (8-wide), 2 wave-coherent (8-wide), 3 per lane (binary)
-    coherent_order: bool = False  # locate: process queries in Morton order
+    coherent_order: bool = False  # locate: process queries in Morton order (False: large unordered batches only)
     mlp: Optional[torch.Tensor] = None   # packed learned initializer (LearnedInitializer.pack())
     mlp_newton_steps: int = 4            # Newton budget from the learned guess before the plain fallback
     start: str = "affine"   # plain Newton start: "affine" (corner-affine estimate) or "centre" (SubRef centre)

@@ -230,6 +230,36 @@ __global__ void __launch_bounds__ (256) k_entry_cells (const uint4 *__restrict__
 // size 1,024 is as good as 64 (4 M, order 3: 3.56 ms against 3.65 ms).
 constexpr int kLocateChunk = 64, kLocateChunkRefill = 128, kLocateChunkLarge = 1024, kLocateRefillRounds = 4;
 
+// Does the order of many points pay for its sort?  Points in no spatial order make every lane of a wavefront read nodes
+// and element nets of its own; sorted, lanes share them.  Sort + walk against walk alone, random points, order 1 / 2 /
+// 3 / 4 on 48^3 elements: 512 K points 0.70 / 0.76 / 1.07 / 1.69x, 1 M 0.96 / 1.08 / 1.48 / 2.29x, 2 M 1.31 / 1.42 /
+// 1.76 / 2.79x, 4 M 1.23 / 1.48 / 2.27 / 4.90x, 16 M 1.52 / 1.92 / 3.10 / 6.43x; much the same from 16^3 to 64^3 (the
+// sort costs about 0.25 ms + 50 us per million points).  Hence the least number of points by order.  On small meshes the
+// lanes share without it: 4 M points on 8^3 elements (16,896 leaves) 0.80 / 1.16 / 1.65 / 2.40x, on 4^3 (2,112 leaves)
+// 0.62 / 0.95 / 1.21 / 1.58x, on 2^3 and 1 down to 0.4x.  Hence the least number of leaves.  The most points bound the
+// sort's scratch (16 bytes each) to 2 GiB.
+static bool order_may_pay (int order, int64_t n, int32_t n_leaves)
+{
+  return n >= (order >= 4 ? 3ll << 17 : order == 3 ? 3ll << 18 : 3ll << 19) && n_leaves >= (order >= 2 ? 1 << 13 : 1 << 16);
+}
+constexpr int64_t kOrderPointsMost = 1ll << 27;
+constexpr int kSpreadWaves = 256;
+
+// Are neighbours in the input neighbours in space already?  Counts, over kSpreadWaves runs of 64 consecutive points spread
+// evenly over the input, the points further than `limit` (a length per axis) from their predecessor.  Points that were
+// sorted, come from rays or from a grid keep their order: they'd gain little from the sort (a 160^3 grid 0 to 30%) or
+// nothing.  16 K points, one launch and a wait (15 us).
+__global__ void __launch_bounds__ (64) k_point_spread (const float *__restrict__ pts, int64_t n, float sx, float sy, float sz,
+                                                       int32_t *__restrict__ far_count)
+{
+  const int lane = threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * ((n - 64) / (kSpreadWaves - 1)) + lane;
+  const float x = pts[3 * i], y = pts[3 * i + 1], z = pts[3 * i + 2];
+  const float dx = fabsf (x - __shfl_up (x, 1)) * sx, dy = fabsf (y - __shfl_up (y, 1)) * sy, dz = fabsf (z - __shfl_up (z, 1)) * sz;
+  const uint64_t b = __ballot (lane > 0 && fmaxf (dx, fmaxf (dy, dz)) > 1.f);
+  if (lane == 0) atomicAdd (far_count, __popcll (b));
+}
+
 // Wave-uniform pool of unclaimed processing-order entries [claimed, end) for the streamed kernels; `more`:
 // further chunks may come from the queue.
 struct EntryPool
@@ -1047,7 +1077,7 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
   int32_t *err = counters ? counters : (int32_t *)arena (SLOT_FLAGS, 64, st);
   if (!err) return DRX_ERR_HIP;
   int32_t *queue = err + 1;   // chunk counter of the persistent launch
-  hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, err, (int64_t)2, 0);
+  hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, err, counters ? (int64_t)2 : (int64_t)3, 0);
   const LocateCfg cfg = make_cfg (mesh, bvh, opts);
   int32_t *steps = opts ? opts->newton_steps : nullptr;
   int32_t *cands = opts ? opts->candidates : nullptr;
@@ -1065,9 +1095,30 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
       if (chunk == 0) chunk = t.chunk;
     }
   }
+  // drx_locate sorts large batches that are in no spatial order (see order_may_pay)
+  const int trav = opts ? opts->traversal : DRX_TRAVERSE_AUTO;
+  const bool by_size = !ws && !given && (trav == DRX_TRAVERSE_AUTO || trav == DRX_TRAVERSE_BINARY || learned) &&
+                       !(opts && opts->coherent_order) && n <= kOrderPointsMost && order_may_pay (mesh->order, n, bvh->n_leaves);
+  bool sort = opts && opts->coherent_order;
+  if (by_size)
+  {
+    // 4 times the larger of the leaves' and the points' own spacing, were they spread evenly
+    const float per_ext = std::cbrt ((float)std::min ((int64_t)std::max (bvh->n_leaves, 1), n)) / 4.f;
+    float scale[3];
+    for (int d = 0; d < 3; ++d)
+    {
+      const float ext = bvh->bounds[2 * d + 1] - bvh->bounds[2 * d];
+      scale[d] = ext > 0.f ? per_ext / ext : 0.f;
+    }
+    hipLaunchKernelGGL (k_point_spread, dim3 (kSpreadWaves), dim3 (64), 0, st, points, n, scale[0], scale[1], scale[2], err + 2);
+    DRX_LAUNCH_CHECK ();
+    int32_t n_far = 0;
+    if (int rc = read_back (&n_far, err + 2, sizeof n_far, st)) return rc;
+    sort = n_far > kSpreadWaves * 63 / 2;
+  }
   const int64_t resident = (int64_t)compute_units (dev) * 4 * locate_waves_per_simd (P, cfg.polish, learned ? 3 : walk);
   // (a chunk of 64 is for small n only, so the grid's work-item count, 64 per chunk, stays in 32 bits)
-  const bool large = n > 64 * kLocateRefillRounds * resident, ordered = learned || (opts && opts->coherent_order);
+  const bool large = n > 64 * kLocateRefillRounds * resident, ordered = learned || by_size || sort;
   if (launch == DRX_LAUNCH_AUTO) launch = large && ordered && chunk == 0 ? DRX_LAUNCH_PERSISTENT : DRX_LAUNCH_CHUNKED;
   if (chunk == 0) chunk = !large ? kLocateChunk : launch == DRX_LAUNCH_PERSISTENT ? kLocateChunkRefill : kLocateChunkLarge;
   if (chunk < 64 || chunk > (1 << 20)) return fail (DRX_ERR_ARG, "drx_locate: chunk %d outside [64, 2^20]", chunk);
@@ -1081,17 +1132,21 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
   const dim3 g (nblk (n, 256)), b (256);
   const dim3 gs ((unsigned)grid_s), bs (64);
   Location *out = (Location *)out_locations;
-  const int trav = opts ? opts->traversal : DRX_TRAVERSE_AUTO;
   if (trav == DRX_TRAVERSE_WAVE && !cfg.wide)
     return fail (DRX_ERR_ARG, "drx_locate: wave traversal needs bvh->wide_nodes");
   // given starts ride on the binary walk
   const int mode = given ? 4 : trav == DRX_TRAVERSE_WAVE ? 2 : (trav == DRX_TRAVERSE_LANE && cfg.wide) ? 1 : 0;
   const int32_t *order = nullptr;
-  if (opts && opts->coherent_order)
+  if (sort)
   {
     if (n > (1ll << 31) - 1) return fail (DRX_ERR_ARG, "drx_locate: coherent_order supports < 2^31 points");
     int rc2 = morton_order_points (points, (int)n, bvh->bounds, st, &order, ws);
-    if (rc2) return rc2;
+    if (rc2 && !by_size) return rc2;
+    if (rc2)
+    {
+      (void)hipGetLastError (); // no room for the sort: the points as they come
+      order = nullptr;
+    }
   }
   const MlpNet net = mlp_net (learned ? opts->mlp : nullptr);
   const int budget = (learned && opts->mlp_newton_steps > 0) ? opts->mlp_newton_steps : 4;

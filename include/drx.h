@@ -140,7 +140,9 @@ typedef struct drx_locate_opts
   int32_t *newton_steps;      /* device, nullable: Newton steps summed over candidates, per point */
   int32_t *candidates;        /* device, nullable: candidate leaves tried, per point */
   int32_t traversal;          /* drx_traversal: how a wavefront walks the BVH (same results either way) */
-  int32_t coherent_order;     /* drx_locate: 1 = process queries in Morton order (results stay in input order) */
+  int32_t coherent_order;     /* drx_locate: 1 = process queries in Morton order (results stay in input order);
+                                 0 = drx_locate does so itself for large batches in no spatial order (plain and
+                                 learned start, binary walk) when its arena has room for 16 bytes per point */
   const void *mlp;            /* DRX_INIT_MLP: packed initializer (drx_mlp_pack), device */
   int32_t mlp_newton_steps;   /* DRX_INIT_MLP: Newton budget from the learned guess before the plain
                                  fallback (<= 0: 4) */
