@@ -344,45 +344,50 @@ __global__ void __launch_bounds__ (256) k_mlp_train (const bf16x8 *__restrict__ 
   }
 }
 
-// partials[w * PSTRIDE + p] summed over rows w0..w1-1 in row order; the loads of eight rows are issued
-// before they are added, so the rows cost one memory latency per eight instead of one each.
+// partials[w * PSTRIDE + p] summed over rows w0..w1-1 in row order; the loads of K rows are issued before they are
+// added, so the rows cost one memory latency per K instead of one each.
+template <int K>
+__device__ __forceinline__ void add_rows (const float *__restrict__ partials, int &w, int w1, int p, float &sum)
+{
+  for (; w + K <= w1; w += K)
+  {
+    float t[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) t[k] = partials[(int64_t)(w + k) * PSTRIDE + p];
+#pragma unroll
+    for (int k = 0; k < K; ++k) sum += t[k];
+  }
+}
+
 __device__ __forceinline__ float ordered_row_sum (const float *__restrict__ partials, int w0, int w1, int p)
 {
   float sum = 0.f;
-  int w = w0;
-  for (; w + 8 <= w1; w += 8)
-  {
-    float t[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) t[k] = partials[(int64_t)(w + k) * PSTRIDE + p];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) sum += t[k];
-  }
-  for (; w < w1; ++w) sum += partials[(int64_t)w * PSTRIDE + p];
+  add_rows<16> (partials, w0, w1, p, sum);
+  add_rows<4> (partials, w0, w1, p, sum);
+  add_rows<1> (partials, w0, w1, p, sum);
   return sum;
 }
 
-// First level of the gradient sum: group g adds its share of the per-block rows, in order.
-constexpr int kGradGroups = 16;
-__global__ void __launch_bounds__ (256) k_mlp_grad_groups (const float *__restrict__ partials, int nwaves,
-                                                           float *__restrict__ groups)
+// Adam over the gradient, then the bf16 copies: 16 threads per parameter add their share of the per-block rows, in order,
+// and the first adds the 16 sums, in order (a fixed order: deterministic).  Thread NPARAM writes the step's mean squared
+// error.  Bound by latency: one round of loads at 256 rows (a batch of 16,384).  32 parameters per block read whole
+// 128-byte lines of a row.  5.3 us against 4.8 + 4.2 us in two launches (group sums, then Adam).
+constexpr int kGradGroups = 16, kAdamParams = 32;
+__global__ void __launch_bounds__ (kGradGroups * kAdamParams) k_mlp_adam (MlpState s, const float *__restrict__ partials,
+                                                                         int nwaves, float lr, float b1, float b2, float eps,
+                                                                         float bc1, float bc2, float loss_scale,
+                                                                         float *__restrict__ loss_out)
 {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > NPARAM) return;
-  const int g = blockIdx.y;
-  const int w0 = (int)((int64_t)nwaves * g / kGradGroups), w1 = (int)((int64_t)nwaves * (g + 1) / kGradGroups);
-  groups[(int64_t)g * PSTRIDE + p] = ordered_row_sum (partials, w0, w1, p);
-}
-
-// Adam over the gradient (the group sums added in a fixed order: deterministic), then the bf16 copies.
-// Thread NPARAM writes the step's mean squared error.
-__global__ void __launch_bounds__ (256) k_mlp_adam (MlpState s, const float *__restrict__ partials, int nwaves, float lr,
-                                                    float b1, float b2, float eps, float bc1, float bc2,
-                                                    float loss_scale, float *__restrict__ loss_out)
-{
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > NPARAM) return;
-  const float gsum = ordered_row_sum (partials, 0, nwaves, p);
+  __shared__ float part[kGradGroups][kAdamParams];
+  const int c = threadIdx.x % kAdamParams, g = threadIdx.x / kAdamParams, p = blockIdx.x * kAdamParams + c;
+  if (p <= NPARAM)
+    part[g][c] = ordered_row_sum (partials, (int)((int64_t)nwaves * g / kGradGroups),
+                                  (int)((int64_t)nwaves * (g + 1) / kGradGroups), p);
+  __syncthreads ();
+  if (g > 0 || p > NPARAM) return;
+  float gsum = 0.f;
+#pragma unroll
+  for (int q = 0; q < kGradGroups; ++q) gsum += part[q][c];
   if (p == NPARAM)
   {
     if (loss_out) *loss_out = gsum * loss_scale;
@@ -540,9 +545,8 @@ int drx_mlp_train (void *state, const void *x, const float *target, int64_t n, c
   if (o->steps < 0) return fail (DRX_ERR_ARG, "drx_mlp_train: negative step count");
   const int nw = o->batch / 64;
   const hipStream_t st = as_stream (stream);
-  float *partials = (float *)arena (SLOT_TREE, (size_t)(nw + kGradGroups) * PSTRIDE * sizeof (float), st);
+  float *partials = (float *)arena (SLOT_TREE, (size_t)nw * PSTRIDE * sizeof (float), st);
   if (!partials) return DRX_ERR_HIP;
-  float *groups = partials + (size_t)nw * PSTRIDE;
   const MlpState s = state_view (state);
   const double b1 = o->beta1 > 0 ? o->beta1 : 0.9, b2 = o->beta2 > 0 ? o->beta2 : 0.999;
   const float eps = o->eps > 0 ? o->eps : 1e-8f;
@@ -558,11 +562,8 @@ int drx_mlp_train (void *state, const void *x, const float *target, int64_t n, c
     // cosine decay from lr to lr_final over total steps
     const double ph = fmin (1.0, (double)(t - 1) / (double)(total > 1 ? total - 1 : 1));
     const float lr = (float)(lr_final + 0.5 * (o->lr - lr_final) * (1.0 + cos (M_PI * ph)));
-    hipLaunchKernelGGL (k_mlp_grad_groups, dim3 ((NPARAM + 1 + 255) / 256, kGradGroups), dim3 (256), 0, st, partials, nw,
-                        groups);
-    DRX_LAUNCH_CHECK ();
-    hipLaunchKernelGGL (k_mlp_adam, dim3 ((NPARAM + 1 + 255) / 256), dim3 (256), 0, st, s, groups, kGradGroups, lr, (float)b1,
-                        (float)b2, eps, (float)(1.0 - pow (b1, t)), (float)(1.0 - pow (b2, t)),
+    hipLaunchKernelGGL (k_mlp_adam, dim3 ((NPARAM + kAdamParams) / kAdamParams),
+                        dim3 (kGradGroups * kAdamParams), 0, st, s, partials, nw, lr, (float)b1, (float)b2, eps, (float)(1.0 - pow (b1, t)), (float)(1.0 - pow (b2, t)),
                         1.f / (float)(o->batch * OUT), out_loss ? out_loss + k : nullptr);
     DRX_LAUNCH_CHECK ();
   }
