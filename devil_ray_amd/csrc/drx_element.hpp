@@ -20,7 +20,6 @@ namespace drx
 
 // Wave-uniform reads through the constant address space become scalar loads.
 typedef const float __attribute__ ((address_space (4))) cfloat;
-typedef const double __attribute__ ((address_space (4))) cdouble;
 
 template <int P> struct Ord
 {
