@@ -880,7 +880,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     return fail (DRX_ERR_ARG, "drx_volume_integrate: %d lights (at most %d, host array)", shading->n_lights,
                  DRX_MAX_LIGHTS);
   *out_count = 0;
-  if (stats) *stats = drx_integrate_stats { 0, 0, 0, 0, 0.f, 0.f, 0 };
+  if (stats) *stats = drx_integrate_stats { 0, 0, 0, 0, 0.f, 0.f, 0, 0 };
   if (n_rays == 0) return DRX_OK;
   if (!active_rays || !out_partials) return fail (DRX_ERR_ARG, "drx_volume_integrate: null rays/output");
   if ((int64_t)n_rays * 5 > (1ll << 31) - 1) return fail (DRX_ERR_ARG, "drx_volume_integrate: too many rays");
@@ -1141,6 +1141,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     stats->kernel_ms = k_ms;
     stats->total_ms = t_ms;
     stats->walk = split ? 5 : mode;
+    stats->binned = split && binned ? 1 : 0;
   }
   return DRX_OK;
 }

@@ -213,6 +213,8 @@ typedef struct drx_integrate_stats
   float total_ms;             /* the whole call: integrate + partial compaction (HIP events) */
   int32_t walk;               /* the walk that ran: 0 binary, 1 8-wide per lane, 2 wave-coherent, 3 learned start,
                                  4 binary with given starts / record, 5 binary walk's candidates, sample-parallel launch */
+  int32_t binned;             /* of the two sample-parallel kernels (walk 5): 1 the one that groups candidates by
+                                 element, 0 the one that locates a sample per lane; 0 for every other walk */
 } drx_integrate_stats;
 
 /* PointLight (rendering/point_light.hpp:15-33); dray's defaults: amb 0.4, diff 0.75, spec 0.8, spec_pow 15. */

@@ -1,0 +1,85 @@
+"""Both sample-parallel kernels against one lane per ray, each on frames that it takes (drx_integrate_stats.binned says
+which ran): the same partials and located, Newton, candidate and polished counts."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from devil_ray_amd import _lib as L
+from devil_ray_amd import synthetic as syn
+from test_gpu_parity import _np, _slab_stack
+
+
+def test_stats_layout():
+    assert L.DrxIntegrateStats.binned.offset == 44 and C.sizeof(L.DrxIntegrateStats) == 48
+
+
+def _compare(gpu, mesh, rays, side, samples, lit, polish, fp64, binned, lights=None, alpha=0.3):
+    vol = gpu.Volume(gpu.UnstructuredMesh(mesh), gpu.UnstructuredField(mesh, fp64=fp64))
+    vol.use_lighting = lit
+    vol.samples(samples)
+    vol.table = gpu.ColorTable()
+    vol.table.add_point(0.0, (0.2, 0.4, 0.9))
+    vol.table.add_point(1.0, (1.0, 0.3, 0.0))
+    vol.table.add_alpha(0.0, alpha)
+    got = {}
+    for launch in (1, 3):
+        vol.opts = gpu.LocateOptions(launch=launch, traversal=3, fp64_polish=polish, cond_threshold=1.0 if polish else 1e4)
+        parts, n = vol.integrate(rays, tile_width=side, tile_height=side, lights=lights)
+        st = vol.last_stats
+        assert (st.walk, st.binned) == ((0, 0) if launch == 1 else (5, binned))
+        got[launch] = ((st.located_samples, st.newton_steps, st.candidates, st.polished), _np(parts, np.uint8)[: n * 24].copy())
+    assert got[1][0][0] > 0 and (not polish or got[1][0][3] > 0)
+    assert got[1][0] == got[3][0]
+    assert np.array_equal(got[1][1], got[3][1])
+    return got[3][1]
+
+
+# Grouped by element: fine meshes, seen along an axis, obliquely (wavefronts whose leaves outgrow the list) and from inside.
+FINE = [
+    ("p1_n16", lambda: syn.hex_mesh(16, 1, 0.05, 0.01, 3), (0.5, 0.5, 3.0), 240, 300, False, False, False),
+    ("p2_n14_fp64_field", lambda: syn.hex_mesh(14, 2, 0.05, 0.01, 5, keep_field64=True), (2.2, 2.0, 2.3), 330, 300, False, False,
+     True),
+    ("p3_n12_lit", lambda: syn.hex_mesh(12, 3, 0.15, 0.01, 4), (-1.4, 1.9, 2.0), 230, 170, True, False, False),
+    ("p4_n10_polish", lambda: syn.hex_mesh(10, 4, 0.2, 0.01, 6), (2.2, 2.0, 2.3), 200, 130, False, True, False),
+    ("mixed_n10", lambda: syn.mixed_hex_mesh(10, 0.1, 0.01, 7), (2.2, 2.0, 2.3), 210, 150, False, False, False),
+    ("p3_n12_inside", lambda: syn.hex_mesh(12, 3, 0.1, 0.01, 8), (0.52, 0.48, 0.55), 120, 160, False, True, False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make,pos,side,samples,lit,polish,fp64", FINE, ids=[c[0] for c in FINE])
+def test_grouped_on_fine_meshes(gpu, name, make, pos, side, samples, lit, polish, fp64):
+    print(f"[grouped] {name}", flush=True)
+    cam = gpu.Camera(side, side, 45.0, pos=pos, look_at=(0.5, 0.5, 0.5))
+    _compare(gpu, make(), cam.create_rays(), side, samples, lit, polish, fp64, 1, [gpu.default_light(cam)])
+
+
+# A sample per lane: fewer than 32 active rays per element column.
+SPARSE = [("p1", lambda: syn.hex_mesh(12, 1, 0.05, 0.01, 11, keep_field64=True)),
+          ("p2", lambda: syn.hex_mesh(12, 2, 0.05, 0.01, 1, keep_field64=True)),
+          ("p3", lambda: syn.hex_mesh(11, 3, 0.1, 0.01, 2, keep_field64=True)),
+          ("p4", lambda: syn.hex_mesh(10, 4, 0.25, 0.01, 3, keep_field64=True)),
+          ("mixed", lambda: syn.mixed_hex_mesh(11, 0.15, 0.05, 5))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make", SPARSE, ids=[c[0] for c in SPARSE])
+def test_sample_per_lane(gpu, name, make):
+    mesh = make()
+    cam = gpu.Camera(40, 40, 45.0, pos=(0.5, 0.6, 2.5), look_at=(0.5, 0.5, 0.5))
+    for lit, polish, fp64, samples in ((False, False, False, 96), (True, False, False, 96), (False, True, False, 96),
+                                       (True, True, False, 64), (False, False, True, 96), (False, True, True, 70),
+                                       (False, False, False, 5)):
+        if fp64 and mesh.field64 is None:
+            continue
+        print(f"[sample per lane] {name} lit={lit} polish={polish} fp64={fp64} samples={samples}", flush=True)
+        _compare(gpu, mesh, cam.create_rays(), 40, samples, lit, polish, fp64, 0, [gpu.default_light(cam)])
+
+
+@pytest.mark.gpu
+def test_sample_per_lane_partial_limit(gpu):
+    rays = syn.orthographic_rays(24, 24)
+    parts = _compare(gpu, _slab_stack(), gpu.as_bytes(rays), 24, 200, False, False, False, 0, alpha=0.02)
+    per_ray = np.bincount(parts.view(syn.PARTIAL_DTYPE)["pixel_id"], minlength=24 * 24)
+    assert (per_ray == 5).sum() > 288 and per_ray.max() == 5
