@@ -181,6 +181,9 @@ constexpr int kWaveWalkMinRaysPerSimd = 48;
 #define DRX_SPLIT_MAX_RAYS_PER_SIMD 300
 #endif
 constexpr int kSplitMaxRaysPerSimd = DRX_SPLIT_MAX_RAYS_PER_SIMD;
+// Samples per ray and round: with 8, groups are small and rounds many (order-3 frame 16.6 ms against 14.2 ms when
+// lanes still walked by themselves; lit frames of eight 6^3 order-2 domains 3.7 ms against 2.3 ms).
+constexpr int kBinnedR = 16;
 // Of the two sample-parallel kernels, the one that bins candidates by element (k_integrate_binned) takes frames with at
 // least this many active rays per element column (rays / elements^(2/3)); with fewer, 64 neighbouring rays cross too
 // many elements to share them.
@@ -188,6 +191,24 @@ constexpr int kSplitMaxRaysPerSimd = DRX_SPLIT_MAX_RAYS_PER_SIMD;
 // 8.6 / 14.0 (93); 40^3 order 4: 4.0 / 3.3 (9), 4.1 / 3.9 (20), 3.3 / 5.1 (46); 56^3 order 2: 3.4 / 3.0 (29); lit 40^3
 // order 3: 1.77 / 1.50 (21), 1.63 / 1.78 (46).
 constexpr double kBinnedMinRaysPerColumn = 32;
+// And where the 64 kBinnedR points of a round, the samples of an 8x8 tile of rays, are expected to put enough of them in each
+// element that they meet: with steps or pixels that are long against an element, groups are small and every point is
+// worked through per lane, 16 samples a round although the ray may end sooner.  The expectation takes a cubic grid of elements
+// over the bounds.  Measured on 810 frames (orders 1-4 and mixed, 6^3 to 48^3 elements, 128^2 to 1100^2 rays, 8 to 600 samples
+// across the bounds, straight and oblique), time of the form that ran otherwise / this one, median and least at
+// points per element: order 1: 0.75, 0.50 (6-12), 0.94, 0.72 (32-40), 1.22, 0.71 (40-50), 1.26, 0.91 (50-60), 1.46 (100-130);
+// order 2: 0.73, 0.50 (6-12), 0.94, 0.70 (32-40), 1.22 (40-50); order 3: 0.75, 0.53 (6-12), 1.03, 0.83 (32-40), 1.32
+// (40-50); order 4: 0.93, 0.67 (12-18), 1.17, 0.94 (24-32); mixed 1-4: 1.00, 0.60 (18-24), 1.11, 0.72 (32-40), 1.24 (40-50).
+static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, const float *bounds6, float sample_dist)
+{
+  double diag2 = 0.0;
+  for (int d = 0; d < 3; ++d) diag2 += ((double)bounds6[2 * d + 1] - bounds6[2 * d]) * ((double)bounds6[2 * d + 1] - bounds6[2 * d]);
+  const double per_axis = std::cbrt ((double)n_el), element = std::sqrt (diag2 / 3.0) / per_axis;
+  const double per_column = n_rays / (per_axis * per_axis);
+  const double across = 1.0 + 8.0 / std::sqrt (per_column), along = 1.0 + kBinnedR * (double)sample_dist / element;
+  const double per_element = 64 * kBinnedR / (across * across * along);
+  return per_column >= kBinnedMinRaysPerColumn && per_element >= 60 - 8 * (order ? order : 3);   // a NaN fails
+}
 constexpr int kIntWaves = kIntBlock / 64;
 
 // SHADE: 0 VolumeShader::color over an FP32 field, 1 shaded_color (lit), 2 color over an FP64 field.
@@ -630,9 +651,6 @@ __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, PO
 // x 200: 9.6 -> 7.1 ms.  Staging the elements in LDS instead of scalar reads: 10.9 and 62 ms.
 // Waves per SIMD: four blocks fit a CU's LDS, three of the lit kernel, whose samples are colours.
 __host__ __device__ constexpr int binned_waves_per_simd (int shade) { return shade == 1 ? 3 : 4; }
-// Samples per ray and round: with 8, groups are small and rounds many (order-3 frame 16.6 ms against 14.2 ms when
-// lanes still walked by themselves; lit frames of eight 6^3 order-2 domains 3.7 ms against 2.3 ms).
-constexpr int kBinnedR = 16;
 
 template <int P, bool POLISH, int SHADE>
 __global__ void __launch_bounds__ (kBinThreads, binned_waves_per_simd (SHADE)) k_integrate_binned (IntegrateArgs a)
@@ -933,7 +951,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   // kSplitMaxRaysPerSimd active rays per SIMD under the automatic walk and launch.
   const int launch = opts ? opts->launch : DRX_LAUNCH_AUTO;
   const bool plain = !guided && !learned && P <= DRX_MAX_MIXED_ORDER;
-  const bool binned = (double)n_rays >= kBinnedMinRaysPerColumn * std::cbrt ((double)mesh->n_el * (double)mesh->n_el);
+  const bool binned = samples_share_elements (P, n_rays, mesh->n_el, bvh->bounds, sample_dist);
   bool split = false;
   if (launch == DRX_LAUNCH_SAMPLES)
   {

@@ -83,3 +83,21 @@ def test_sample_per_lane_partial_limit(gpu):
     parts = _compare(gpu, _slab_stack(), gpu.as_bytes(rays), 24, 200, False, False, False, 0, alpha=0.02)
     per_ray = np.bincount(parts.view(syn.PARTIAL_DTYPE)["pixel_id"], minlength=24 * 24)
     assert (per_ray == 5).sum() > 288 and per_ray.max() == 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", [1, 2, 3, 4, 0])
+def test_coarse_march_per_lane(gpu, p):
+    """Steps as long as an element: the form that ran before candidates were grouped, in small and in large frames."""
+    n = 14 if p < 4 else 13
+    mesh = syn.hex_mesh(n, p, 0.05, 0.01, 3) if p else syn.mixed_hex_mesh(n, 0.1, 0.01, 3)
+    cam = gpu.Camera(200, 200, 45.0, pos=(2.2, 2.0, 2.3), look_at=(0.5, 0.5, 0.5))
+    _compare(gpu, mesh, cam.create_rays(), 200, 8, False, False, False, 0)
+    vol = gpu.Volume(gpu.UnstructuredMesh(mesh), gpu.UnstructuredField(mesh))
+    vol.use_lighting = False
+    side = 640
+    for samples, want in ((8, (0, 0)), (400, (5, 1))):
+        vol.samples(samples)
+        vol.integrate(gpu.Camera(side, side, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.5, 0.5, 0.0)).create_rays(), tile_width=side,
+                      tile_height=side)
+        assert (vol.last_stats.walk, vol.last_stats.binned) == want, samples
