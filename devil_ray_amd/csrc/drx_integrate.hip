@@ -24,6 +24,8 @@ struct IntegrateArgs
   const int64_t *field_offsets;
   const Ray *rays;
   const int32_t *order;
+  const int32_t *choice;       // of two forms launched one after the other, the one with use == *choice gets the
+  int32_t use;                 // rays (k_integrate_choice).  (Beside err they would be loaded with it and held.)
   int n_rays;
   const float4 *lut;
   int lut_size;
@@ -38,6 +40,10 @@ struct IntegrateArgs
   int n_lights;                // lit shading (LIT kernels)
   drx_point_light lights[DRX_MAX_LIGHTS];
 };
+
+// The number of rays for a kernel of which another form was launched too: all of them or none.  (With a return
+// at its start k_integrate_binned spills two more scalar registers, then a vector register: 1.4% of a frame.)
+__device__ __forceinline__ int rays_here (const IntegrateArgs &a) { return *a.choice == a.use ? a.n_rays : 0; }
 
 // A pointer for lanes' own elements (UNI false) or for one element per wavefront, read by scalar loads.
 template <bool UNI, typename T> __device__ __forceinline__ auto element_ptr (const T *p)
@@ -195,10 +201,12 @@ constexpr double kBinnedMinRaysPerColumn = 32;
 // element that they meet: with steps or pixels that are long against an element, groups are small and every point is
 // worked through per lane, 16 samples a round although the ray may end sooner.  The expectation takes a cubic grid of elements
 // over the bounds.  Measured on 810 frames (orders 1-4 and mixed, 6^3 to 48^3 elements, 128^2 to 1100^2 rays, 8 to 600 samples
-// across the bounds, straight and oblique), time of the form that ran otherwise / this one, median and least at
-// points per element: order 1: 0.75, 0.50 (6-12), 0.94, 0.72 (32-40), 1.22, 0.71 (40-50), 1.26, 0.91 (50-60), 1.46 (100-130);
-// order 2: 0.73, 0.50 (6-12), 0.94, 0.70 (32-40), 1.22 (40-50); order 3: 0.75, 0.53 (6-12), 1.03, 0.83 (32-40), 1.32
-// (40-50); order 4: 0.93, 0.67 (12-18), 1.17, 0.94 (24-32); mixed 1-4: 1.00, 0.60 (18-24), 1.11, 0.72 (32-40), 1.24 (40-50).
+// across the bounds, straight and oblique), time of the form that ran otherwise / this one at points per element, least and
+// median: up to 6: 0.50, 0.65 (orders 1, 2), 0.52, 0.72 (order 3), 0.56, 0.82 (order 4); 12-24: 0.54, 0.91 (1, 2), 0.64, 0.96
+// (3), 0.57, 1.0 (4).  Of those whose rays lie together (k_integrate_choice): orders 1, 2: 1.33 (37), 0.94 (38), 1.29 to 1.57 (43-46),
+// 1.16 to 1.2 (49-56); order 3: 0.85 (16), 0.98 (21), 0.87 to 1.15 (29-33), 1.39 (37), 1.03 (38), 1.44 (43); order 4: 0.93 (16),
+// 1.06 to 1.31 (21), 0.88 to 1.39 (29-33), 1.11 (38), 1.55 (43); mixed 1-4: 0.88 (16), 1.01 (21), 0.96 to 1.07 (29), 1.49 (37).
+constexpr double kBinnedMinPoints = 36, kBinnedMinPointsOrder4 = 20;
 static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, const float *bounds6, float sample_dist)
 {
   double diag2 = 0.0;
@@ -207,8 +215,62 @@ static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, con
   const double per_column = n_rays / (per_axis * per_axis);
   const double across = 1.0 + 8.0 / std::sqrt (per_column), along = 1.0 + kBinnedR * (double)sample_dist / element;
   const double per_element = 64 * kBinnedR / (across * across * along);
-  return per_column >= kBinnedMinRaysPerColumn && per_element >= 60 - 8 * (order ? order : 3);   // a NaN fails
+  return per_column >= kBinnedMinRaysPerColumn && per_element >= (order == 4 ? kBinnedMinPointsOrder4 : kBinnedMinPoints);   // a NaN fails
 }
+// Do the rays of a block lie together?  Grouping pays where a wavefront finds its points' leaves by one descent and they
+// share elements: not for rays in no order or without the tile order, nor for small frames seen so obliquely that the box
+// around a wavefront's points is mostly empty.  Four wavefronts look at 64 consecutive rays of the processing order each, at
+// an eighth, three, five and seven eighths of it: the box around four consecutive samples of theirs half way along
+// the longest of the rays, in leaves (spread evenly over the bounds).  With three of the four boxes within the limit the
+// frame takes the grouping kernel (choice 1).  One block, in the place of the launch that clears the counters.  Up to
+// kChoiceWaitRays rays both forms are launched and one of them finds no rays (65,536 rays: 6 to 8 us); above, the host waits for
+// the choice (14 us) and launches one.
+//
+// The limit by measurement, as above: time of the other form / of this one, least, median and most at leaves in the third
+// smallest box.  Against the per-lane sample-parallel form, order 1: 1.07, 1.31, 1.66 (up to 20), 1.09, 1.36, 1.46 (30-40), 0.78,
+// 1.00, 1.04 (60-70), 1.04, 1.09 (80-100), 0.76, 0.83, 0.86 (100-300); order 2: 1.19, 1.46, 1.81 (up to 20), 1.07, 1.11, 1.13
+// (60-70), 1.22, 1.28 (80-100), 0.79, 0.92, 1.03 (100-300); order 3: 1.39, 1.40 (80-100), 0.88, 1.07, 1.17 (150-300); order 4: 0.88,
+// 0.95, 1.04 (100-112), 1.02, 1.23, 1.53 (150-300), 0.86, 1.19, 1.38 (300-500); mixed 1-4: 1.11, 1.36, 1.65 (150-300).  Against
+// one lane per ray, orders 1-3: 0.91, 1.21, 1.33 (112-200).  Rays in no order have thousands.
+constexpr float kBoxLeavesLowOrders = 100.f, kBoxLeaves = 300.f;
+constexpr int32_t kChoiceWaitRays = 1 << 18;
+
+__global__ void __launch_bounds__ (256) k_integrate_choice (const Ray *__restrict__ rays, const int32_t *__restrict__ order, int n_rays,
+                                                            float sample_dist, float sx, float sy, float sz, float most_leaves,
+                                                            int32_t *__restrict__ counters, int n_counters, int32_t *choice)
+{
+  __shared__ int32_t fit;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (threadIdx.x == 0) fit = 0;
+  if ((int)threadIdx.x < n_counters) counters[threadIdx.x] = 0;
+  __syncthreads ();
+  const int64_t tile = ((int64_t)n_rays + 63) / 64 * (2 * wv + 1) / 8, i = 64 * tile + lane;
+  const bool has_ray = i < n_rays;
+  Ray ray = rays[has_ray ? (order ? order[i] : i) : 0];
+  const float half = 0.5f * wave_reduce_max (has_ray ? ray.far_ - ray.near_ : 0.f);
+  float lo[3] = { INFINITY, INFINITY, INFINITY }, hi[3] = { -INFINITY, -INFINITY, -INFINITY };
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+  {
+    const float t = ray.near_ + half + q * sample_dist;
+    if (has_ray && t - sample_dist < ray.far_)
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+      {
+        const float x = ray_point (ray.orig[d], t, ray.dir[d]);
+        lo[d] = fminf (lo[d], x);
+        hi[d] = fmaxf (hi[d], x);
+      }
+  }
+  const float scale[3] = { sx, sy, sz };
+  float leaves = 1.f;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) leaves *= 1.f + fmaxf (wave_reduce_max (hi[d]) - wave_reduce_min (lo[d]), 0.f) * scale[d];
+  if (lane == 0 && leaves <= most_leaves) atomicAdd (&fit, 1);
+  __syncthreads ();
+  if (threadIdx.x == 0) *choice = fit >= 3 ? 1 : 0;
+}
+
 constexpr int kIntWaves = kIntBlock / 64;
 
 // SHADE: 0 VolumeShader::color over an FP32 field, 1 shaded_color (lit), 2 color over an FP64 field.
@@ -242,7 +304,7 @@ __global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) 
   todo.bdim = blockDim.x;
   todo.tid = threadIdx.x;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool has_ray = t < a.n_rays;
+  const bool has_ray = t < (MODE == 0 ? rays_here (a) : a.n_rays);
   unsigned long long located = 0;
   LocateStats st { 0, 0, 0, 0 };
   bool overflow = false;
@@ -456,6 +518,7 @@ constexpr int32_t kSplitFound = 1 << 30, kSplitPolished = 1 << 29, kSplitOverflo
 template <int P, bool POLISH, int SHADE>
 __global__ void __launch_bounds__ (64 * kSplitWaves, split_waves_per_simd (P, POLISH)) k_integrate_split (IntegrateArgs a)
 {
+  if (*a.choice != a.use) return;
   __shared__ int32_t stack_lds[kStackLds * 64 * kSplitWaves];
   __shared__ float4 rcol[kSplitR * 64];   // sample colours, [sample of the round][lane]
   __shared__ int2 rcnt[kSplitR * 64];     // Newton steps; candidates | found / polished / overflow bits
@@ -664,7 +727,7 @@ __global__ void __launch_bounds__ (kBinThreads, binned_waves_per_simd (SHADE)) k
   __shared__ int32_t more;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int i = blockIdx.x * 64 + lane;
-  const bool has_ray = i < a.n_rays;
+  const bool has_ray = i < rays_here (a);
   const int ri = has_ray ? (a.order ? a.order[i] : i) : 0;
   Ray ray;
   if (has_ray)
@@ -910,8 +973,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   unsigned long long *dstats = (unsigned long long *)arena (SLOT_STATS, 8 * sizeof (unsigned long long), st);
   if (!slots || !counts || !dstats) return DRX_ERR_HIP;
   int32_t *first = counts + n_blocks;
-  int32_t *err = (int32_t *)(dstats + 4);
-  hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)16, 0);
+  int32_t *err = (int32_t *)(dstats + 4);   // overflow flag, number of partials, choice of the form
   IntegrateArgs a;
   a.cfg = make_cfg (mesh, bvh, opts);
   a.cfg.polished_out = nullptr;   // per-point flags belong to batched locate
@@ -938,6 +1000,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   a.slots = slots;
   a.stats = dstats;
   a.err = err;
+  a.choice = err + 2;
   a.net = mlp_net (learned ? opts->mlp : nullptr);
   a.budget = (learned && opts->mlp_newton_steps > 0) ? opts->mlp_newton_steps : 4;
   a.n_lights = lit ? shading->n_lights : 0;
@@ -947,27 +1010,26 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   const int trav = opts ? opts->traversal : DRX_TRAVERSE_AUTO;
   if (trav == DRX_TRAVERSE_WAVE && !a.cfg.wide)
     return fail (DRX_ERR_ARG, "drx_volume_integrate: wave traversal needs bvh->wide_nodes");
-  // Sample-parallel launch (k_integrate_split): asked for, or picked for frames of fewer than
-  // kSplitMaxRaysPerSimd active rays per SIMD under the automatic walk and launch.
+  // Sample-parallel launch: asked for, or picked for frames of fewer than kSplitMaxRaysPerSimd active rays per SIMD
+  // under the automatic walk and launch.  In its place, and in the place of one lane per ray, frames whose samples share
+  // elements take k_integrate_binned, but for small BVHs that carry the 8-wide copy (the wave walk) in large frames.
   const int launch = opts ? opts->launch : DRX_LAUNCH_AUTO;
   const bool plain = !guided && !learned && P <= DRX_MAX_MIXED_ORDER;
-  const bool binned = samples_share_elements (P, n_rays, mesh->n_el, bvh->bounds, sample_dist);
-  bool split = false;
+  bool split = false, binned = false;
   if (launch == DRX_LAUNCH_SAMPLES)
   {
     if (!plain || (trav != DRX_TRAVERSE_AUTO && trav != DRX_TRAVERSE_BINARY))
       return fail (DRX_ERR_UNSUPPORTED, "drx_volume_integrate: the sample-parallel launch runs the binary walk with "
                    "the plain start, orders up to %d", DRX_MAX_MIXED_ORDER);
-    split = true;
+    split = binned = true;
   }
   else if (launch == DRX_LAUNCH_AUTO && trav == DRX_TRAVERSE_AUTO && plain)
   {
-    // large frames too where the rays are dense, but for small BVHs that carry the 8-wide copy (the wave walk)
     int dev = 0;
-    split = hipGetDevice (&dev) == hipSuccess &&
-            ((int64_t)n_rays < (int64_t)kSplitMaxRaysPerSimd * 4 * compute_units (dev) ||
-             (binned && !(a.cfg.wide && bvh->n_leaves <= kWaveWalkMaxLeaves)));
+    split = hipGetDevice (&dev) == hipSuccess && (int64_t)n_rays < (int64_t)kSplitMaxRaysPerSimd * 4 * compute_units (dev);
+    binned = split || !(a.cfg.wide && bvh->n_leaves <= kWaveWalkMaxLeaves);
   }
+  binned = binned && samples_share_elements (P, n_rays, mesh->n_el, bvh->bounds, sample_dist);
   int walk = split ? DRX_TRAVERSE_BINARY : trav;
   if (walk == DRX_TRAVERSE_AUTO && a.cfg.wide && !learned && P <= DRX_MAX_MIXED_ORDER)
   {
@@ -984,9 +1046,6 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   if (P > DRX_MAX_MIXED_ORDER && mode != 0)
     return fail (DRX_ERR_UNSUPPORTED, "drx_volume_integrate: order %d runs the binary walk with the plain start "
                  "only (orders up to %d take the other forms)", P, DRX_MAX_MIXED_ORDER);
-  hipEvent_t ev[3];
-  for (int q = 0; q < 3; ++q) DRX_HIP (hipEventCreate (&ev[q]));
-  DRX_HIP (hipEventRecord (ev[0], st));
 #define DRX_INT2(PP, PO, LT)                                             \
   do                                                                     \
   {                                                                      \
@@ -1055,80 +1114,114 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     else                                                                                   \
       hipLaunchKernelGGL ((k_integrate_binned<PP, PO, 0>), gs, bs, 0, st, a);              \
   } while (0)
-  if (split && binned)
-  {
-    if (a.cfg.polish)
+  const auto march = [&] (bool grouped) {
+    a.use = grouped ? 1 : 0;
+    if (grouped)
+    {
+      if (a.cfg.polish)
+        switch (P)
+        {
+        case 0: DRX_BINNED (0, true); break;
+        case 1: DRX_BINNED (1, true); break;
+        case 2: DRX_BINNED (2, true); break;
+        case 3: DRX_BINNED (3, true); break;
+        default: DRX_BINNED (4, true); break;
+        }
+      else
+        switch (P)
+        {
+        case 0: DRX_BINNED (0, false); break;
+        case 1: DRX_BINNED (1, false); break;
+        case 2: DRX_BINNED (2, false); break;
+        case 3: DRX_BINNED (3, false); break;
+        default: DRX_BINNED (4, false); break;
+        }
+    }
+    else if (split)
+    {
+      if (a.cfg.polish)
+        switch (P)
+        {
+        case 0: DRX_SPLIT (0, true); break;
+        case 1: DRX_SPLIT (1, true); break;
+        case 2: DRX_SPLIT (2, true); break;
+        case 3: DRX_SPLIT (3, true); break;
+        default: DRX_SPLIT (4, true); break;
+        }
+      else
+        switch (P)
+        {
+        case 0: DRX_SPLIT (0, false); break;
+        case 1: DRX_SPLIT (1, false); break;
+        case 2: DRX_SPLIT (2, false); break;
+        case 3: DRX_SPLIT (3, false); break;
+        default: DRX_SPLIT (4, false); break;
+        }
+    }
+    else if (a.cfg.polish)
       switch (P)
       {
-      case 0: DRX_BINNED (0, true); break;
-      case 1: DRX_BINNED (1, true); break;
-      case 2: DRX_BINNED (2, true); break;
-      case 3: DRX_BINNED (3, true); break;
-      default: DRX_BINNED (4, true); break;
+      case 0: DRX_INT (0, true); break;
+      case 1: DRX_INT (1, true); break;
+      case 2: DRX_INT (2, true); break;
+      case 3: DRX_INT (3, true); break;
+      case 4: DRX_INT (4, true); break;
+      case 5: DRX_INT_HI (5, true); break;
+      case 6: DRX_INT_HI (6, true); break;
+      case 7: DRX_INT_HI (7, true); break;
+      default: DRX_INT_HI (8, true); break;
       }
     else
       switch (P)
       {
-      case 0: DRX_BINNED (0, false); break;
-      case 1: DRX_BINNED (1, false); break;
-      case 2: DRX_BINNED (2, false); break;
-      case 3: DRX_BINNED (3, false); break;
-      default: DRX_BINNED (4, false); break;
+      case 0: DRX_INT (0, false); break;
+      case 1: DRX_INT (1, false); break;
+      case 2: DRX_INT (2, false); break;
+      case 3: DRX_INT (3, false); break;
+      case 4: DRX_INT (4, false); break;
+      case 5: DRX_INT_HI (5, false); break;
+      case 6: DRX_INT_HI (6, false); break;
+      case 7: DRX_INT_HI (7, false); break;
+      default: DRX_INT_HI (8, false); break;
       }
-  }
-  else if (split)
-  {
-    if (a.cfg.polish)
-      switch (P)
-      {
-      case 0: DRX_SPLIT (0, true); break;
-      case 1: DRX_SPLIT (1, true); break;
-      case 2: DRX_SPLIT (2, true); break;
-      case 3: DRX_SPLIT (3, true); break;
-      default: DRX_SPLIT (4, true); break;
-      }
-    else
-      switch (P)
-      {
-      case 0: DRX_SPLIT (0, false); break;
-      case 1: DRX_SPLIT (1, false); break;
-      case 2: DRX_SPLIT (2, false); break;
-      case 3: DRX_SPLIT (3, false); break;
-      default: DRX_SPLIT (4, false); break;
-      }
-  }
-  else if (a.cfg.polish)
-    switch (P)
-    {
-    case 0: DRX_INT (0, true); break;
-    case 1: DRX_INT (1, true); break;
-    case 2: DRX_INT (2, true); break;
-    case 3: DRX_INT (3, true); break;
-    case 4: DRX_INT (4, true); break;
-    case 5: DRX_INT_HI (5, true); break;
-    case 6: DRX_INT_HI (6, true); break;
-    case 7: DRX_INT_HI (7, true); break;
-    default: DRX_INT_HI (8, true); break;
-    }
-  else
-    switch (P)
-    {
-    case 0: DRX_INT (0, false); break;
-    case 1: DRX_INT (1, false); break;
-    case 2: DRX_INT (2, false); break;
-    case 3: DRX_INT (3, false); break;
-    case 4: DRX_INT (4, false); break;
-    case 5: DRX_INT_HI (5, false); break;
-    case 6: DRX_INT_HI (6, false); break;
-    case 7: DRX_INT_HI (7, false); break;
-    default: DRX_INT_HI (8, false); break;
-    }
+  };
 #undef DRX_INT_HI
 #undef DRX_SPLIT
 #undef DRX_BINNED
 #undef DRX_INT
 #undef DRX_INT64
 #undef DRX_INT2
+  hipEvent_t ev[3];
+  for (int q = 0; q < 3; ++q) DRX_HIP (hipEventCreate (&ev[q]));
+  const int n_counters = 16;
+  if (binned)
+  {
+    float scale[3];
+    const float per_axis = std::cbrt ((float)bvh->n_leaves);
+    for (int d = 0; d < 3; ++d)
+    {
+      const float ext = bvh->bounds[2 * d + 1] - bvh->bounds[2 * d];
+      scale[d] = ext > 0.f ? per_axis / ext : 0.f;
+    }
+    const float most = split && (P == 1 || P == 2) ? kBoxLeavesLowOrders : kBoxLeaves;
+    hipLaunchKernelGGL (k_integrate_choice, dim3 (1), dim3 (256), 0, st, a.rays, a.order, n_rays, sample_dist, scale[0], scale[1],
+                        scale[2], most, (int32_t *)dstats, n_counters, err + 2);
+  }
+  else
+    hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)n_counters, 0);
+  DRX_LAUNCH_CHECK ();
+  bool both = binned;
+  if (binned && n_rays > kChoiceWaitRays)
+  {
+    int32_t choice = 0;
+    if ((rc = read_back (&choice, err + 2, sizeof choice, st))) return rc;
+    binned = choice == 1;
+    both = false;
+  }
+  DRX_HIP (hipEventRecord (ev[0], st));
+  if (binned) march (true);
+  DRX_LAUNCH_CHECK ();
+  if (!binned || both) march (false);
   DRX_LAUNCH_CHECK ();
   DRX_HIP (hipEventRecord (ev[1], st));
   DRX_LAUNCH_CHECK ();
@@ -1143,6 +1236,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   unsigned long long hs[8];
   if ((rc = read_back (hs, dstats, sizeof hs, st))) return rc;
   const int32_t total = ((int32_t *)(hs + 4))[1];
+  binned = binned && ((int32_t *)(hs + 4))[2] == 1;
   float k_ms = 0.f, t_ms = 0.f;
   DRX_HIP (hipEventElapsedTime (&k_ms, ev[0], ev[1]));
   DRX_HIP (hipEventElapsedTime (&t_ms, ev[0], ev[2]));
@@ -1158,8 +1252,8 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     stats->polished = (int64_t)hs[3];
     stats->kernel_ms = k_ms;
     stats->total_ms = t_ms;
-    stats->walk = split ? 5 : mode;
-    stats->binned = split && binned ? 1 : 0;
+    stats->walk = split || binned ? 5 : mode;
+    stats->binned = binned ? 1 : 0;
   }
   return DRX_OK;
 }

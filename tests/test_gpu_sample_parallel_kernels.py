@@ -101,3 +101,31 @@ def test_coarse_march_per_lane(gpu, p):
         vol.integrate(gpu.Camera(side, side, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.5, 0.5, 0.0)).create_rays(), tile_width=side,
                       tile_height=side)
         assert (vol.last_stats.walk, vol.last_stats.binned) == want, samples
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,p,side", [(12, 3, 300), (14, 2, 640)])
+def test_rays_in_no_order_per_lane(gpu, n, p, side):
+    """The form is chosen by how the rays lie in processing order: grouped in tile order; a sample (small frame) or a ray
+    (more than 300 active rays per SIMD) per lane for the same rays shuffled.  The partials of a ray are the same."""
+    mesh = syn.hex_mesh(n, p, 0.1, 0.01, 4)
+    m = gpu.UnstructuredMesh(mesh)
+    vol = gpu.Volume(m, gpu.UnstructuredField(mesh))
+    vol.use_lighting = False
+    vol.samples(200)
+    vol.table = gpu.ColorTable()
+    vol.table.add_alpha(0.0, 0.3)
+    cam = gpu.Camera(side, side, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.4, 0.45, 0.0))
+    act, k = gpu.remove_missed_rays(cam.create_rays(), m.bounds())
+    rays = _np(act, np.uint8)[: k * 36].reshape(k, 36)
+    perm = np.random.default_rng(3).permutation(k)
+    parts, cnt = vol.integrate(None, tile_width=side, tile_height=side, active=(act, k))
+    assert (vol.last_stats.walk, vol.last_stats.binned) == (5, 1)
+    counts = (vol.last_stats.newton_steps, vol.last_stats.candidates)
+    a = _np(parts, np.uint8)[: cnt * 24].view(syn.PARTIAL_DTYPE)
+    parts, cnt2 = vol.integrate(None, active=(gpu.as_bytes(rays[perm].copy()), k))
+    assert (vol.last_stats.walk, vol.last_stats.binned) == (5 if side < 500 else 0, 0)
+    assert counts == (vol.last_stats.newton_steps, vol.last_stats.candidates)
+    b = _np(parts, np.uint8)[: cnt2 * 24].view(syn.PARTIAL_DTYPE)
+    assert cnt == cnt2
+    assert np.array_equal(np.sort(a, order=["pixel_id", "depth"]).view(np.uint8), np.sort(b, order=["pixel_id", "depth"]).view(np.uint8))
