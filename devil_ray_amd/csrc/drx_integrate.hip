@@ -232,16 +232,25 @@ static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, con
 // (60-70), 1.22, 1.28 (80-100), 0.79, 0.92, 1.03 (100-300); order 3: 1.39, 1.40 (80-100), 0.88, 1.07, 1.17 (150-300); order 4: 0.88,
 // 0.95, 1.04 (100-112), 1.02, 1.23, 1.53 (150-300), 0.86, 1.19, 1.38 (300-500); mixed 1-4: 1.11, 1.36, 1.65 (150-300).  Against
 // one lane per ray, orders 1-3: 0.91, 1.21, 1.33 (112-200).  Rays in no order have thousands.
+//
+// And can rays end early?  A round locates 16 samples of a ray whether or not it is opaque after two.  Where a colour table's
+// largest opacity lets a ray end within kSamplesToEnd samples the other forms stay.  Time of the other form / of this one, least
+// and median over 213 frames with one opacity for all samples, by the samples after which a ray ends: 4: 0.30, 0.88; 8: 0.30,
+// 1.01; 14: 0.86, 1.17; 20: 0.70, 1.03; 28: 0.88, 1.18; 40: 0.85, 1.29; 64: 0.80, 1.21.  (The default table, opacity 0.7 per ten
+// samples of a hundred, ends a ray after 25 at the earliest; up to 90 samples, where it may end one sooner, the forms are within
+// 12% of each other on eight domains of 4^3 to 10^3 elements.)
+constexpr int kSamplesToEnd = 24;
 constexpr float kBoxLeavesLowOrders = 100.f, kBoxLeaves = 300.f;
 constexpr int32_t kChoiceWaitRays = 1 << 18;
 
 __global__ void __launch_bounds__ (256) k_integrate_choice (const Ray *__restrict__ rays, const int32_t *__restrict__ order, int n_rays,
                                                             float sample_dist, float sx, float sy, float sz, float most_leaves,
+                                                            const float4 *__restrict__ lut, int lut_size, float opacity,
                                                             int32_t *__restrict__ counters, int n_counters, int32_t *choice)
 {
-  __shared__ int32_t fit;
+  __shared__ int32_t fit, opaque;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (threadIdx.x == 0) fit = 0;
+  if (threadIdx.x == 0) fit = opaque = 0;
   if ((int)threadIdx.x < n_counters) counters[threadIdx.x] = 0;
   __syncthreads ();
   const int64_t tile = ((int64_t)n_rays + 63) / 64 * (2 * wv + 1) / 8, i = 64 * tile + lane;
@@ -267,8 +276,11 @@ __global__ void __launch_bounds__ (256) k_integrate_choice (const Ray *__restric
 #pragma unroll
   for (int d = 0; d < 3; ++d) leaves *= 1.f + fmaxf (wave_reduce_max (hi[d]) - wave_reduce_min (lo[d]), 0.f) * scale[d];
   if (lane == 0 && leaves <= most_leaves) atomicAdd (&fit, 1);
+  bool ends = false;
+  for (int q = threadIdx.x; q < lut_size; q += 256) ends = ends || !(lut[q].w < opacity);   // a NaN is none to rely on
+  if (ends) atomicOr (&opaque, 1);
   __syncthreads ();
-  if (threadIdx.x == 0) *choice = fit >= 3 ? 1 : 0;
+  if (threadIdx.x == 0) *choice = fit >= 3 && !opaque ? 1 : 0;
 }
 
 constexpr int kIntWaves = kIntBlock / 64;
@@ -1205,7 +1217,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     }
     const float most = split && (P == 1 || P == 2) ? kBoxLeavesLowOrders : kBoxLeaves;
     hipLaunchKernelGGL (k_integrate_choice, dim3 (1), dim3 (256), 0, st, a.rays, a.order, n_rays, sample_dist, scale[0], scale[1],
-                        scale[2], most, (int32_t *)dstats, n_counters, err + 2);
+                        scale[2], most, a.lut, lut_size, 1.f - std::pow (0.05f, 1.f / kSamplesToEnd), (int32_t *)dstats, n_counters, err + 2);
   }
   else
     hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)n_counters, 0);

@@ -129,3 +129,23 @@ def test_rays_in_no_order_per_lane(gpu, n, p, side):
     b = _np(parts, np.uint8)[: cnt2 * 24].view(syn.PARTIAL_DTYPE)
     assert cnt == cnt2
     assert np.array_equal(np.sort(a, order=["pixel_id", "depth"]).view(np.uint8), np.sort(b, order=["pixel_id", "depth"]).view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opacity,grouped", [(0.10, 1), (0.13, 0), (1.0, 0)])
+@pytest.mark.parametrize("lit", [False, True])
+def test_opaque_tables_per_lane(gpu, opacity, grouped, lit):
+    """A colour table with which a ray can end within 24 samples (opacity per sample 1 - 0.05^(1/24) = 0.117) keeps the form
+    that works a sample, or in frames of more than 300 active rays per SIMD a ray, per lane."""
+    mesh = syn.hex_mesh(14, 2, 0.05, 0.01, 3)
+    alpha = 1.0 - (1.0 - opacity) ** 20.0   # the table is corrected by 10 / samples
+    cam = gpu.Camera(120, 120, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.5, 0.5, 0.0))
+    _compare(gpu, mesh, cam.create_rays(), 120, 200, lit, False, False, grouped, [gpu.default_light(cam)], alpha)
+    vol = gpu.Volume(gpu.UnstructuredMesh(mesh), gpu.UnstructuredField(mesh))
+    vol.use_lighting = lit
+    vol.samples(200)
+    vol.table = gpu.ColorTable()
+    vol.table.add_alpha(0.0, alpha)
+    cam = gpu.Camera(640, 640, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.5, 0.5, 0.0))
+    vol.integrate(cam.create_rays(), tile_width=640, tile_height=640, lights=[gpu.default_light(cam)])
+    assert (vol.last_stats.walk, vol.last_stats.binned) == ((5, 1) if grouped else (0, 0))
