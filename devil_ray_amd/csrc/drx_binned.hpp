@@ -33,7 +33,10 @@ constexpr int kBinMin = 32;
 constexpr int kBinLeaves = 112;
 constexpr int kBinProbes = 8;
 typedef TravStackOf<0> BinStack;              // of a lane that walks by itself (rare): no LDS
-// A point's record: Newton steps (17 bits), candidates (12 bits, counted up to 4,095), flags.
+// A point that has tried this many candidates is left: it is not for this form, where a round of few points leaves most of the
+// block idle and a point that walks by itself starts its walk anew in every round.
+constexpr int kBinCands = 128;
+// A point's record: Newton steps (17 bits), candidates (12 bits), flags.
 constexpr uint32_t kRecSteps = (1u << 17) - 1, kRecCandOne = 1u << 17, kRecCands = 0xFFFu << 17, kRecOverflow = 1u << 29,
                    kRecFound = 1u << 30, kRecPolished = 1u << 31;
 // What follows a point's candidate: a leaf (>= 0), nothing, a candidate that only a walk finds, or an entry of a
@@ -43,6 +46,7 @@ constexpr int32_t kNextNone = -1, kNextWalk = -2, kNextList = -16;   // kNextLis
 constexpr int32_t kNextMore = 1 << 12, kNextScan = 1 << 13, kNextEntry = (1 << 12) - 1;
 constexpr int32_t kLeafMore = 1 << 30;   // on a leaf: further hits, found by a walk
 static_assert (kBinWaves * kBinLeaves <= kNextEntry, "list entries fit their bits");
+static_assert (kBinCands <= (int)(kRecCands / kRecCandOne) && kBinCands * 20 <= (int)kRecSteps, "counts fit their bits");
 
 // A leaf of a wavefront's list: exact box, element and leaf index.
 struct BinLeaf
@@ -216,7 +220,7 @@ __device__ __forceinline__ void bin_hits (const BinLeaf *list, int n, const floa
 //   accept (item, el, ref, uni): called by one lane for a located item (uni: std::true_type when el is uniform);
 //   span: sets of 64 points per leaf list where one list cannot hold those of all sets (Q / 2 at first, halved when
 //   a list overflows, kept by the caller between calls).
-// Leaves sh.rec[item]; ends with a barrier.
+// Leaves sh.rec[item] (with kBinCands candidates and not found: perhaps unfinished); ends with a barrier.
 template <int P, bool POLISH, int N, typename OwnPoint, typename Point, typename Accept>
 __device__ __forceinline__ void locate_binned (const LocateCfg &cfg, BinShared<N> &sh, int &span, OwnPoint &&own_point,
                                                Point &&point, Accept &&accept)
@@ -463,11 +467,9 @@ __device__ __forceinline__ void locate_binned (const LocateCfg &cfg, BinShared<N
           if (found) accept (item, el, x, std::false_type ());
         }
         uint32_t c = sh.rec[item];
-        const uint32_t steps = (c & kRecSteps) + (uint32_t)st.newton;
-        c = (c & ~kRecSteps) | (steps < kRecSteps ? steps : kRecSteps);
-        if ((c & kRecCands) != kRecCands) c += kRecCandOne;
+        c += kRecCandOne + (uint32_t)st.newton;
         sh.rec[item] = c | (found ? kRecFound : 0) | (st.polished ? kRecPolished : 0);
-        if (!found) sh.next[atomicAdd (&sh.n_next, 1)] = (uint16_t)item;
+        if (!found && (c & kRecCands) < kBinCands * kRecCandOne) sh.next[atomicAdd (&sh.n_next, 1)] = (uint16_t)item;
       }
     }
     sh.key[tid] = -1;   // read again only behind the next round's barrier

@@ -847,7 +847,7 @@ __global__ void __launch_bounds__ (kBinThreads, binned_waves_per_simd (SHADE)) k
         v[1] += cn & kRecSteps;
         v[2] += (cn & kRecCands) / kRecCandOne;
         v[3] += (cn & kRecPolished) ? 1 : 0;
-        if (cn & kRecOverflow)
+        if (!(cn & kRecFound) && (cn & (kRecOverflow | kRecCands)) >= kBinCands * kRecCandOne)   // unfinished
         {
           overflow = true;
           alive = false;
@@ -1235,25 +1235,37 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   DRX_LAUNCH_CHECK ();
   if (!binned || both) march (false);
   DRX_LAUNCH_CHECK ();
-  DRX_HIP (hipEventRecord (ev[1], st));
-  DRX_LAUNCH_CHECK ();
-  hipLaunchKernelGGL (k_count_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots, counts);
-  DRX_LAUNCH_CHECK ();
-  const bool scanned = n_blocks > kCompactSelfScan;
-  if (scanned && (rc = exclusive_scan_i32 (counts, first, n_blocks, nullptr, st))) return rc;
-  hipLaunchKernelGGL (k_compact_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots,
-                      scanned ? first : counts, scanned, err + 1, (Partial *)out_partials);
-  DRX_LAUNCH_CHECK ();
-  DRX_HIP (hipEventRecord (ev[2], st));
   unsigned long long hs[8];
-  if ((rc = read_back (hs, dstats, sizeof hs, st))) return rc;
-  const int32_t total = ((int32_t *)(hs + 4))[1];
-  binned = binned && ((int32_t *)(hs + 4))[2] == 1;
+  const auto finish = [&] () -> int {
+    DRX_HIP (hipEventRecord (ev[1], st));
+    hipLaunchKernelGGL (k_count_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots, counts);
+    DRX_LAUNCH_CHECK ();
+    const bool scanned = n_blocks > kCompactSelfScan;
+    if (scanned)
+      if (int r = exclusive_scan_i32 (counts, first, n_blocks, nullptr, st)) return r;
+    hipLaunchKernelGGL (k_compact_partials, dim3 (n_blocks), dim3 (kCompactThreads), 0, st, slots, n_slots,
+                        scanned ? first : counts, scanned, err + 1, (Partial *)out_partials);
+    DRX_LAUNCH_CHECK ();
+    DRX_HIP (hipEventRecord (ev[2], st));
+    return read_back (hs, dstats, sizeof hs, st);
+  };
+  const int32_t *host_err = (const int32_t *)(hs + 4);
+  if ((rc = finish ())) return rc;
+  binned = binned && host_err[2] == 1;
+  if (binned && host_err[0])   // a sample that the grouping form left unfinished (kBinCands): the other form decides
+  {
+    binned = false;
+    hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)n_counters, 0);
+    march (false);
+    DRX_LAUNCH_CHECK ();
+    if ((rc = finish ())) return rc;
+  }
+  const int32_t total = host_err[1];
   float k_ms = 0.f, t_ms = 0.f;
   DRX_HIP (hipEventElapsedTime (&k_ms, ev[0], ev[1]));
   DRX_HIP (hipEventElapsedTime (&t_ms, ev[0], ev[2]));
   for (int q = 0; q < 3; ++q) (void)hipEventDestroy (ev[q]);
-  if (((int32_t *)(hs + 4))[0])
+  if (host_err[0])
     return fail (DRX_ERR_OVERFLOW, "drx_volume_integrate: BVH traversal stack (%d entries) overflowed", kStackDepth);
   *out_count = total;
   if (stats)

@@ -207,7 +207,7 @@ typedef struct drx_integrate_stats
 {
   int64_t located_samples;    /* successful locate() calls inside the march */
   int64_t newton_steps;       /* Newton iterations over all candidates */
-  int64_t candidates;         /* candidate leaves tried (sample-parallel launch: up to 4,095 counted a sample) */
+  int64_t candidates;         /* candidate leaves tried */
   int64_t polished;           /* samples that took the FP64 correction */
   float kernel_ms;            /* duration of the integrate kernel alone (HIP events on `stream`) */
   float total_ms;             /* the whole call: integrate + partial compaction (HIP events) */

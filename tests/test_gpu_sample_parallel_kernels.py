@@ -149,3 +149,22 @@ def test_opaque_tables_per_lane(gpu, opacity, grouped, lit):
     cam = gpu.Camera(640, 640, 60.0, pos=(0.5, 0.5, 0.95), look_at=(0.5, 0.5, 0.0))
     vol.integrate(cam.create_rays(), tile_width=640, tile_height=640, lights=[gpu.default_light(cam)])
     assert (vol.last_stats.walk, vol.last_stats.binned) == ((5, 1) if grouped else (0, 0))
+
+
+@pytest.mark.gpu
+def test_many_candidates_counted(gpu):
+    """2,200 thin slabs on the diagonal of one small box: a sample beside their plane is in more than 4,095 leaf boxes and
+    in no element. The frame is left to the form that counts them all."""
+    slab = syn.box_net((0.0, 0.0, -1e-3), (0.14, 0.1, 1e-3), 1)
+    c = np.sqrt(0.5)
+    slab = slab @ np.array([[c, 0.0, c], [0.0, 1.0, 0.0], [-c, 0.0, c]]) + [0.45, 0.45, 0.45]
+    nets = [slab] * 2200 + [syn.box_net((x, y, z), (x + 0.1, y + 0.4, z + 0.1), 1)
+                            for x in (0.0, 0.9) for y in (0.0, 0.6) for z in (0.0, 0.9)]
+    field = np.random.default_rng(1).uniform(0, 1, (len(nets), 8))
+    mesh = syn.elements_from_nets(np.stack(nets), 1, field=field)
+    side = 96
+    g = (np.arange(side) + 0.5) / side
+    rays = syn.orthographic_rays(side, side)
+    rays["orig"][:, 0], rays["orig"][:, 1], rays["orig"][:, 2] = np.tile(g, side), -0.5, np.repeat(g, side)
+    rays["dir"] = (1e-7, 1.0, 1e-7)
+    _compare(gpu, mesh, gpu.as_bytes(rays), side, 160, False, False, False, 0, alpha=0.2)
