@@ -34,7 +34,8 @@ class DrxMesh(C.Structure):
 class DrxBVH(C.Structure):
     _fields_ = [("inner_nodes", P), ("leaf_nodes", P), ("aabb_ids", P), ("subrefs", P), ("leaf_pack", P),
                 ("wide_nodes", P), ("n_leaves", I32), ("bounds", F32 * 6), ("leaf_starts", P), ("qnodes", P),
-                ("leaf_boxes", P), ("qgrid", F32 * 6), ("entry_cells", P), ("entry_bits", I32 * 3)]
+                ("leaf_boxes", P), ("qgrid", F32 * 6), ("entry_cells", P), ("entry_bits", I32 * 3),
+                ("entry_mark", C.c_uint32)]
 
 
 class DrxLocateOpts(C.Structure):
@@ -84,6 +85,7 @@ _SIGS = {
     "drx_bvh_pack_leaves": (I32, [C.POINTER(DrxBVH), P, P]),
     "drx_bvh_leaf_starts": (I32, [C.POINTER(DrxMesh), C.POINTER(DrxBVH), P, P]),
     "drx_bvh_entry_bits": (I64, [I32, P, P]),
+    "drx_bvh_entry_mark": (C.c_uint32, [C.POINTER(DrxBVH)]),
     "drx_bvh_entry_cells": (I32, [C.POINTER(DrxBVH), P, P, P]),
     "drx_bvh_quantize": (I32, [C.POINTER(DrxBVH), P, P, P, P]),
     "drx_locate_autotune": (I32, [C.POINTER(DrxMesh), C.POINTER(DrxBVH), P, I64, P, C.POINTER(DrxLocateOpts),

@@ -100,6 +100,7 @@ class BVH:
             if self.entry_cells is not None:
                 v.entry_cells = self.entry_cells.data_ptr()
                 v.entry_bits[:] = [int(b) for b in self.entry_bits]
+                v.entry_mark = L.lib().drx_bvh_entry_mark(C.byref(v))
         return v
 
     def quantize(self) -> None:

@@ -237,6 +237,7 @@ template <class ElemT> drx_bvh UnstructuredMesh<ElemT>::bvh_view ()
     {
       v.entry_cells = m_bvh.m_entry_cells.get_device_ptr_const ();
       for (int d = 0; d < 3; ++d) v.entry_bits[d] = m_bvh.m_entry_bits[d];
+      v.entry_mark = drx_bvh_entry_mark (&v);
     }
   }
   return v;

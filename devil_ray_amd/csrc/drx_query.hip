@@ -1042,6 +1042,20 @@ int64_t drx_bvh_entry_bits (int32_t n_leaves, const float *bounds6, int32_t *out
   return (int64_t)1 << (out_bits[0] + out_bits[1] + out_bits[2]);
 }
 
+uint32_t drx_bvh_entry_mark (const drx_bvh *bvh)
+{
+  if (!bvh) return 0;
+  uint64_t h = 0x9E3779B97F4A7C15ull;
+  for (const uint64_t v : { (uint64_t)(uintptr_t)bvh->qnodes, (uint64_t)(uintptr_t)bvh->entry_cells,
+                            (uint64_t)(uint32_t)bvh->n_leaves << 32 | (uint32_t)bvh->entry_bits[0],
+                            (uint64_t)(uint32_t)bvh->entry_bits[1] << 32 | (uint32_t)bvh->entry_bits[2] })
+  {
+    h = (h ^ v) * 0xBF58476D1CE4E5B9ull;
+    h ^= h >> 31;
+  }
+  return (uint32_t)(h >> 32) | 1u;   // never that of cleared memory
+}
+
 int drx_bvh_entry_cells (const drx_bvh *bvh, const int32_t *bits, uint32_t *out_cells, void *stream)
 {
   if (!bvh || !bvh->qnodes || bvh->n_leaves < 2 || !bits || !out_cells)

@@ -189,13 +189,18 @@ static inline int check_mesh (const drx_mesh *m, int ncomp, const char *what)
   return DRX_OK;
 }
 
+// Whether the entry members were set by a caller that knows them (they came after the others, and a struct that a caller
+// fills member by member need not be clear).
+static inline bool has_entry_cells (const drx_bvh *b) { return b->entry_cells && b->entry_mark == drx_bvh_entry_mark (b); }
+
 static inline int check_bvh (const drx_bvh *b, const char *what)
 {
   if (!b || !b->inner_nodes || !b->leaf_pack) return fail (DRX_ERR_ARG, "%s: bvh needs inner_nodes and leaf_pack", what);
   if (b->n_leaves < 2) return fail (DRX_ERR_ARG, "%s: bvh has %d leaves (dray pads to >= 2)", what, b->n_leaves);
-  if (b->entry_cells)
+  if (has_entry_cells (b))
     for (int d = 0; d < 3; ++d)
-      if (b->entry_bits[d] < 0 || b->entry_bits[d] > 16) return fail (DRX_ERR_ARG, "%s: bvh entry_bits", what);
+      if (b->entry_bits[d] < 0 || b->entry_bits[d] > 16 || b->entry_bits[0] + b->entry_bits[1] + b->entry_bits[2] > 30)
+        return fail (DRX_ERR_ARG, "%s: bvh entry_bits", what);
   return DRX_OK;
 }
 
@@ -213,7 +218,7 @@ static inline LocateCfg make_cfg (const drx_mesh *m, const drx_bvh *b, const drx
     c.q_inv[d] = b->qgrid[3 + d];
   }
   if (c.qnodes && !c.leaf_boxes) c.qnodes = nullptr;
-  c.entry = c.qnodes ? (const uint4 *)b->entry_cells : nullptr;
+  c.entry = c.qnodes && has_entry_cells (b) ? (const uint4 *)b->entry_cells : nullptr;
   for (int d = 0; d < 3; ++d) c.entry_bits[d] = c.entry ? b->entry_bits[d] : 0;
   c.centre = o && (o->init_mode == DRX_INIT_SUBREF_CENTRE || (o->init_mode == DRX_INIT_MLP && o->mlp_fallback == 1));
   c.starts = c.centre ? nullptr : (const float4 *)b->leaf_starts;

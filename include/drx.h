@@ -110,7 +110,10 @@ typedef struct drx_bvh
   float qgrid[6];             /* with qnodes: grid origin xyz, grid cells per unit length xyz */
   const uint32_t *entry_cells;/* optional, with qnodes: entry cells of the binary walk (drx_bvh_entry_cells) */
   int32_t entry_bits[3];      /* with entry_cells: 2^bits cells along x, y, z */
-} drx_bvh;                    /* zero the struct before filling it in: members left out are then not used */
+  uint32_t entry_mark;        /* with entry_cells: drx_bvh_entry_mark of the struct with everything else set.  The
+                                 entry members are used only with it, so that a caller that knows nothing of them
+                                 need not clear them */
+} drx_bvh;
 
 /* Location (location.hpp:16-21): {int32 cell (-1 = not found), float ref[3]} = 16 bytes. */
 /* Ray (ray.hpp:20-28): {float dir[3], near, orig[3], far; int32 pixel_id} = 36 bytes.   */
@@ -313,6 +316,8 @@ int drx_bvh_quantize (const drx_bvh *bvh, uint32_t *out_qnodes, float *out_leaf_
  * bounds and returns the number of cells; out_cells: 4 words per cell.  Needs n_leaves, qnodes, qgrid. */
 int64_t drx_bvh_entry_bits (int32_t n_leaves, const float *bounds6, int32_t *out_bits);
 int drx_bvh_entry_cells (const drx_bvh *bvh, const int32_t *bits, uint32_t *out_cells, void *stream);
+/* The entry_mark of a drx_bvh whose n_leaves, qnodes, entry_cells and entry_bits are set (host). */
+uint32_t drx_bvh_entry_mark (const drx_bvh *bvh);
 /* 8-wide traversal copy of the binary BVH: children in binary left-to-right order, exact float boxes,
  * so traversal visits the same candidate leaves in the same order as dray's binary depth-first walk.
  * Node = 64 floats: lo_x[8] lo_y[8] lo_z[8] hi_x[8] hi_y[8] hi_z[8] child[8] (int32 bits) pad[8].
