@@ -55,6 +55,8 @@ enum ArenaSlot
   SLOT_COUNT
 };
 void *arena (int slot, size_t bytes, hipStream_t stream);   // nullptr + error set on failure
+void arena_free (int slot, hipStream_t stream);             // gives a slot's buffer back in stream order
+void clear_error ();                                        // of a failure that the call goes on without
 // Copies a few bytes from the device to the host, in stream order, and waits for them.
 int read_back (void *host, const void *device, size_t bytes, hipStream_t stream);
 int arena_release ();
@@ -105,16 +107,17 @@ int radix_sort_pairs (uint32_t *kA, int32_t *vA, uint32_t *kB, int32_t *vB, int3
 int radix_tiles (int n);
 inline int64_t radix_hist_len (int n) { return 2 * 256 * (int64_t)radix_tiles (n) + 8; }
 
-// Caller-provided buffers for morton_order_points (n keys/values each, hist and scan sums as above).
+// Buffers of morton_order_points (n keys/values each, hist and scan sums as above).
 struct SortScratch
 {
   uint32_t *kA, *kB;
   int32_t *vA, *vB, *hist, *scan_sums;
 };
-// Permutation of n query points in Morton order over bounds6 (host); lives in `ws` when given, else in
-// the arena's sort slots.
+int sort_scratch (int n, hipStream_t st, SortScratch *out);   // from the arena's sort slots
+void sort_scratch_free (hipStream_t st);                      // gives those back
+// Permutation of n query points in Morton order over bounds6 (host); lives in `ws`.
 int morton_order_points (const float *pts, int n, const float *bounds6, hipStream_t st, const int32_t **order_out,
-                         const SortScratch *ws = nullptr);
+                         const SortScratch &ws);
 
 // Resolves the current device's address of drx_locate_noalloc's static scratch array (once per device).
 int locate_noalloc_setup ();

@@ -1000,24 +1000,26 @@ __global__ void k_point_morton (const float *__restrict__ pts, int n, float minx
   vals[i] = i;
 }
 
-int morton_order_points (const float *pts, int n, const float *bounds6, hipStream_t st, const int32_t **order_out,
-                         const SortScratch *ws)
+int sort_scratch (int n, hipStream_t st, SortScratch *out)
 {
-  uint32_t *kA, *kB;
-  int32_t *vA, *vB, *hist, *sums = nullptr;
-  if (ws)
-  {
-    kA = ws->kA, kB = ws->kB, vA = ws->vA, vB = ws->vB, hist = ws->hist, sums = ws->scan_sums;
-  }
-  else
-  {
-    kA = (uint32_t *)arena (SLOT_SORT_KEYS_A, sizeof (uint32_t) * (size_t)n, st);
-    kB = (uint32_t *)arena (SLOT_SORT_KEYS_B, sizeof (uint32_t) * (size_t)n, st);
-    vA = (int32_t *)arena (SLOT_SORT_VALS_A, sizeof (int32_t) * (size_t)n, st);
-    vB = (int32_t *)arena (SLOT_SORT_VALS_B, sizeof (int32_t) * (size_t)n, st);
-    hist = (int32_t *)arena (SLOT_SORT_HIST, sizeof (int32_t) * (size_t)radix_hist_len (n), st);
-  }
-  if (!kA || !kB || !vA || !vB || !hist) return DRX_ERR_HIP;
+  out->kA = (uint32_t *)arena (SLOT_SORT_KEYS_A, sizeof (uint32_t) * (size_t)n, st);
+  out->kB = out->kA ? (uint32_t *)arena (SLOT_SORT_KEYS_B, sizeof (uint32_t) * (size_t)n, st) : nullptr;
+  out->vA = out->kB ? (int32_t *)arena (SLOT_SORT_VALS_A, sizeof (int32_t) * (size_t)n, st) : nullptr;
+  out->vB = out->vA ? (int32_t *)arena (SLOT_SORT_VALS_B, sizeof (int32_t) * (size_t)n, st) : nullptr;
+  out->hist = out->vB ? (int32_t *)arena (SLOT_SORT_HIST, sizeof (int32_t) * (size_t)radix_hist_len (n), st) : nullptr;
+  out->scan_sums = out->hist ? (int32_t *)arena (SLOT_SCAN, sizeof (int32_t) * (size_t)scan_sums_len (256 * radix_tiles (n)), st)
+                             : nullptr;
+  return out->scan_sums ? DRX_OK : DRX_ERR_HIP;
+}
+
+void sort_scratch_free (hipStream_t st)
+{
+  for (int s : { SLOT_SORT_KEYS_A, SLOT_SORT_KEYS_B, SLOT_SORT_VALS_A, SLOT_SORT_VALS_B, SLOT_SORT_HIST }) arena_free (s, st);
+}
+
+int morton_order_points (const float *pts, int n, const float *bounds6, hipStream_t st, const int32_t **order_out,
+                         const SortScratch &ws)
+{
   float minc[3], inv[3];
   for (int d = 0; d < 3; ++d)
   {
@@ -1026,11 +1028,11 @@ int morton_order_points (const float *pts, int n, const float *bounds6, hipStrea
     inv[d] = (ext > 0.f) ? 1.f / ext : 0.f;
   }
   hipLaunchKernelGGL (k_point_morton, dim3 (nblk (n, 256)), dim3 (256), 0, st, pts, n, minc[0], minc[1], minc[2], inv[0],
-                      inv[1], inv[2], kA, vA);
+                      inv[1], inv[2], ws.kA, ws.vA);
   DRX_LAUNCH_CHECK ();
   uint32_t *ks;
   int32_t *vs;
-  int rc = radix_sort_pairs (kA, vA, kB, vB, hist, n, kPointMortonBits, st, &ks, &vs, sums);
+  int rc = radix_sort_pairs (ws.kA, ws.vA, ws.kB, ws.vB, ws.hist, n, kPointMortonBits, st, &ks, &vs, ws.scan_sums);
   if (rc) return rc;
   *order_out = vs;
   return DRX_OK;

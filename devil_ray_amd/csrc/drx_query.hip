@@ -1154,13 +1154,17 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
   if (sort)
   {
     if (n > (1ll << 31) - 1) return fail (DRX_ERR_ARG, "drx_locate: coherent_order supports < 2^31 points");
-    int rc2 = morton_order_points (points, (int)n, bvh->bounds, st, &order, ws);
-    if (rc2 && !by_size) return rc2;
-    if (rc2)
-    {
-      (void)hipGetLastError (); // no room for the sort: the points as they come
-      order = nullptr;
-    }
+    SortScratch own;
+    if (!ws)
+      if (int rc = sort_scratch ((int)n, st, &own))
+      {
+        if (!by_size) return rc;
+        sort_scratch_free (st);   // no room for a sort that the caller did not ask for: the points as they come
+        clear_error ();
+        sort = false;
+      }
+    if (sort)
+      if (int rc = morton_order_points (points, (int)n, bvh->bounds, st, &order, ws ? *ws : own)) return rc;
   }
   const MlpNet net = mlp_net (learned ? opts->mlp : nullptr);
   const int budget = (learned && opts->mlp_newton_steps > 0) ? opts->mlp_newton_steps : 4;

@@ -27,6 +27,12 @@ void set_error (const char *fmt, ...)
   g_last_error = buf;
 }
 
+void clear_error ()
+{
+  (void)hipGetLastError ();
+  g_last_error.clear ();
+}
+
 int fail (int status, const char *fmt, ...)
 {
   char buf[1024];
@@ -105,6 +111,16 @@ void *arena (int slot, size_t bytes, hipStream_t stream)
   }
   s.bytes = want;
   return s.ptr;
+}
+
+void arena_free (int slot, hipStream_t stream)
+{
+  int dev = 0;
+  if (hipGetDevice (&dev) != hipSuccess) return;
+  std::lock_guard<std::mutex> lock (g_arena_mutex);
+  Slot &s = slot_set (dev, stream).slots[slot];
+  if (s.ptr) (void)hipFreeAsync (s.ptr, stream);
+  s = Slot {};
 }
 
 // A few bytes from the device to the host, and the wait for them.  They land in a pinned word block that the stream's

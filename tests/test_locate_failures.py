@@ -1,0 +1,67 @@
+"""drx_locate's own sort where its memory or a launch fails (on the CPU, over tests/fake_hip.c): without room for the sort
+the points are taken as they come, nothing is kept and no error is left; a failing launch is reported."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+N = 3 << 18   # enough points of order 3 for the sort
+
+CHILD = r"""
+import ctypes as C, json, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+from devil_ray_amd import _lib as L
+lib = L.lib()
+get = lambda n, t=C.c_int: t.in_dll(fake, n)
+get("fake_fail_malloc").value, get("fake_fail_launch").value = int(sys.argv[3]), int(sys.argv[4])
+get("fake_first_copy").value = 1 << 20
+n = int(sys.argv[5])
+buf = C.create_string_buffer(64)
+at = C.addressof(buf)
+m, b, o = L.DrxMesh(), L.DrxBVH(), L.DrxLocateOpts()
+m.data, m.n_el, m.order, m.ncomp, m.stride = at, 1000, 3, 3, lib.drx_mesh_stride(3, 3)
+b.inner_nodes = b.leaf_pack = b.leaf_nodes = b.aabb_ids = b.subrefs = at
+b.n_leaves = 33000
+b.bounds[:] = [0, 1, 0, 1, 0, 1]
+o.coherent_order = int(sys.argv[6])
+rc = lib.drx_locate(C.byref(m), C.byref(b), at, n, at, C.byref(o), None)
+print(json.dumps([rc, (lib.drx_last_error() or b"").decode(), get("fake_mallocs").value, get("fake_launches").value,
+                  get("fake_live", C.c_long).value]))
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-O1", "-Wall", os.path.join(HERE, "fake_hip.c"), "-o", so])
+    return so
+
+
+def _run(fake, fail_malloc=-1, fail_launch=-1, n=N, coherent=0):
+    r = subprocess.run([sys.executable, "-c", CHILD, fake, os.path.dirname(HERE), str(fail_malloc), str(fail_launch), str(n),
+                        str(coherent)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.strip().splitlines()[-1])
+
+
+def test_no_room_for_the_sort(fake):
+    rc, text, mallocs, launches, live = _run(fake)
+    assert (rc, text) == (0, "") and mallocs == 7 and live >= 16 * N   # flags, the sort's six
+    for k in range(1, mallocs):
+        rc, text, got, fewer, live = _run(fake, fail_malloc=k)
+        assert (rc, text) == (0, "") and got == k + 1 and fewer < launches and live < 4 * N, k
+        # asked for, the sort is not left out
+        rc, text, _, _, _ = _run(fake, fail_malloc=k, coherent=1)
+        assert rc == 2 and "out of memory" in text, k
+
+
+def test_failing_launch_is_reported(fake):
+    _, _, _, launches, _ = _run(fake)
+    assert launches > 8
+    for k in range(launches):
+        rc, text, _, _, _ = _run(fake, fail_launch=k)
+        assert rc == 2 and "launch" in text, k
