@@ -237,9 +237,12 @@ constexpr int kLocateChunk = 64, kLocateChunkRefill = 128, kLocateChunkLarge = 1
 // sort costs about 0.25 ms + 50 us per million points).  Hence the least number of points by order.  On small meshes the
 // lanes share without it: 4 M points on 8^3 elements (16,896 leaves) 0.80 / 1.16 / 1.65 / 2.40x, on 4^3 (2,112 leaves)
 // 0.62 / 0.95 / 1.21 / 1.58x, on 2^3 and 1 down to 0.4x.  Hence the least number of leaves.  The most points bound the
-// sort's scratch (16 bytes each) to 2 GiB.
-static bool order_may_pay (int order, int64_t n, int32_t n_leaves)
+// sort's scratch (16 bytes each) to 2 GiB.  A mesh of mixed orders is known by its largest order only; it takes order 3's
+// line at most: of orders 1 to 4 in equal parts 400 K points 0.85, 600 K 1.04, 800 K 1.05, 1.2 M 1.75x, 97% order 1: 0.74, 0.94,
+// 1.02, 1.85x, 95% order 3: 0.95, 1.16, 1.26, 1.9x (16^3 to 48^3 elements, the sort against input order).
+static bool order_may_pay (const drx_mesh *mesh, int64_t n, int32_t n_leaves)
 {
+  const int order = mesh->elem_order ? std::min (mesh->order, 3) : mesh->order;
   return n >= (order >= 4 ? 3ll << 17 : order == 3 ? 3ll << 18 : 3ll << 19) && n_leaves >= (order >= 2 ? 1 << 13 : 1 << 16);
 }
 constexpr int64_t kOrderPointsMost = 1ll << 27;
@@ -1112,7 +1115,7 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
   // drx_locate sorts large batches that are in no spatial order (see order_may_pay)
   const int trav = opts ? opts->traversal : DRX_TRAVERSE_AUTO;
   const bool by_size = !ws && !given && (trav == DRX_TRAVERSE_AUTO || trav == DRX_TRAVERSE_BINARY || learned) &&
-                       !(opts && opts->coherent_order) && n <= kOrderPointsMost && order_may_pay (mesh->order, n, bvh->n_leaves);
+                       !(opts && opts->coherent_order) && n <= kOrderPointsMost && order_may_pay (mesh, n, bvh->n_leaves);
   bool sort = opts && opts->coherent_order;
   if (by_size)
   {

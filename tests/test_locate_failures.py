@@ -1,5 +1,6 @@
-"""drx_locate's own sort where its memory or a launch fails (on the CPU, over tests/fake_hip.c): without room for the sort
-the points are taken as they come, nothing is kept and no error is left; a failing launch is reported."""
+"""When drx_locate sorts by itself, and what it does where the sort's memory or a launch fails (on the CPU, over
+tests/fake_hip.c): without room for the sort the points are taken as they come, nothing is kept and no error is left; a
+failing launch is reported."""
 import json
 import os
 import subprocess
@@ -28,6 +29,9 @@ b.inner_nodes = b.leaf_pack = b.leaf_nodes = b.aabb_ids = b.subrefs = at
 b.n_leaves = 33000
 b.bounds[:] = [0, 1, 0, 1, 0, 1]
 o.coherent_order = int(sys.argv[6])
+if int(sys.argv[7]):   # mixed orders
+    m.elem_order = m.elem_offset = at
+    m.order, m.stride = int(sys.argv[7]), 0
 rc = lib.drx_locate(C.byref(m), C.byref(b), at, n, at, C.byref(o), None)
 print(json.dumps([rc, (lib.drx_last_error() or b"").decode(), get("fake_mallocs").value, get("fake_launches").value,
                   get("fake_live", C.c_long).value]))
@@ -41,9 +45,9 @@ def fake(tmp_path_factory):
     return so
 
 
-def _run(fake, fail_malloc=-1, fail_launch=-1, n=N, coherent=0):
+def _run(fake, fail_malloc=-1, fail_launch=-1, n=N, coherent=0, mixed=0):
     r = subprocess.run([sys.executable, "-c", CHILD, fake, os.path.dirname(HERE), str(fail_malloc), str(fail_launch), str(n),
-                        str(coherent)], capture_output=True, text=True, timeout=120)
+                        str(coherent), str(mixed)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-2000:]
     return json.loads(r.stdout.strip().splitlines()[-1])
 
@@ -65,3 +69,10 @@ def test_failing_launch_is_reported(fake):
     for k in range(launches):
         rc, text, _, _, _ = _run(fake, fail_launch=k)
         assert rc == 2 and "launch" in text, k
+
+
+@pytest.mark.parametrize("order,least", [(4, 3 << 18), (3, 3 << 18), (2, 3 << 19)])
+def test_mixed_orders_sort_from(fake, order, least):
+    """A mesh of mixed orders whose largest is 4 is not taken for one of order 4: most of its elements may be of order 1."""
+    assert _run(fake, n=least - 1, mixed=order)[2] == 1   # the flags alone
+    assert _run(fake, n=least, mixed=order)[2] == 7
