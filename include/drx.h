@@ -145,7 +145,8 @@ typedef struct drx_locate_opts
   int32_t traversal;          /* drx_traversal: how a wavefront walks the BVH (same results either way) */
   int32_t coherent_order;     /* drx_locate: 1 = process queries in Morton order (results stay in input order);
                                  0 = drx_locate does so itself for large batches in no spatial order (plain and
-                                 learned start, binary walk) when its arena has room for 16 bytes per point */
+                                 learned start, binary walk) when its arena has room for 16 bytes per point, which
+                                 it keeps for the next batch until drx_release; drx_locate_noalloc never does */
   const void *mlp;            /* DRX_INIT_MLP: packed initializer (drx_mlp_pack), device */
   int32_t mlp_newton_steps;   /* DRX_INIT_MLP: Newton budget from the learned guess before the plain
                                  fallback (<= 0: 4) */
@@ -178,8 +179,8 @@ enum drx_launch
                                  them (same partials and statistics; binary walk, plain start, orders up to
                                  DRX_MAX_MIXED_ORDER).  Under DRX_LAUNCH_AUTO and DRX_TRAVERSE_AUTO a render
                                  takes it for frames of fewer than 300 active rays per SIMD, and for larger
-                                 ones of at least 32 active rays per element column unless the wave walk
-                                 applies; DRX_LAUNCH_CHUNKED or DRX_LAUNCH_PERSISTENT keep one lane per ray */
+                                 ones whose samples share elements (drx_integrate_stats.binned) unless the wave
+                                 walk applies; DRX_LAUNCH_CHUNKED or DRX_LAUNCH_PERSISTENT keep one lane per ray */
 };
 
 /* Training schedule of the learned initializer (drx_mlp_train): Adam, cosine decay lr -> lr_final over
@@ -217,7 +218,11 @@ typedef struct drx_integrate_stats
   int32_t walk;               /* the walk that ran: 0 binary, 1 8-wide per lane, 2 wave-coherent, 3 learned start,
                                  4 binary with given starts / record, 5 binary walk's candidates, sample-parallel launch */
   int32_t binned;             /* of the two sample-parallel kernels (walk 5): 1 the one that groups candidates by
-                                 element, 0 the one that locates a sample per lane; 0 for every other walk */
+                                 element, 0 the one that locates a sample per lane; 0 for every other walk.  The
+                                 first runs where neighbouring samples share elements: at least 32 active rays per
+                                 element column, steps and pixels short against an element, 64 consecutive rays of
+                                 the processing order lying together, no ray opaque within 24 samples, no sample
+                                 with 128 candidates */
 } drx_integrate_stats;
 
 /* PointLight (rendering/point_light.hpp:15-33); dray's defaults: amb 0.4, diff 0.75, spec 0.8, spec_pow 15. */
