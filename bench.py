@@ -9,9 +9,11 @@ opacity 0.02, unlit.  One step = one frame: camera rays -> remove_missed_rays ->
 integrate (locate + field eval + LUT + blend, <= 5 partials/ray) -> partial compaction -> composite.
 
 Prints one JSON line.  value = located samples/s over the whole frame (inputs resident in HBM).
-roofline: the integrate kernel, algorithmic bytes = 16 B x (p+1)^3 per located sample (fp32
-geometry + field of the located element, one compulsory fetch, no reuse; 20 B x (p+1)^3 for the 8^3
-order-2 frame, whose scalar field is FP64), timed with HIP events on the stream the kernel runs on.  cpu_baseline: the CPU oracle (dray's OpenMP path restated) on a
+roofline: the integrate kernel, timed with HIP events on the stream it runs on.  Where it groups candidates by
+element (one scalar read of a control net serves a group of samples) it is bound by the vector units: FP32
+operations of the Newton steps and field evaluations against their rate without packed FP32.  The other forms:
+algorithmic bytes = 16 B x (p+1)^3 per located sample (fp32 geometry + field of the located element, one fetch, no
+reuse; 20 B x (p+1)^3 with an FP64 field) against HBM.  cpu_baseline: the CPU oracle (dray's OpenMP path restated) on a
 bounded, evenly spread subset of the same frame's active rays, timed on this host's cores.
 """
 from __future__ import annotations
@@ -29,11 +31,18 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+FP32_PEAK_TFLOPS = 78.6   # 256 CUs x 4 SIMDs x 16 lanes x 2 per multiply-add x 2.4 GHz, no packed FP32
 # HBM bytes per launch of the dominant kernel, from two rocprofv3 --pmc runs (FETCH_SIZE, then WRITE_SIZE)
 # scaled by what the counters read for a 1 GiB device copy (x2.0, x1.0); the summary with its commands is
 # profiles/k_integrate_binned_p3_64cubed_1024sq_512spp.md.  Keyed by (config, kernel) so that other workloads or
 # kernel variants report null rather than a stale figure.
 PMC_TRAFFIC_BYTES = {(1, "k_integrate_binned<3,false,0>"): 6.03e9 + 1.22e9}
+
+
+def _newton_flops(p: int) -> int:
+    """One evaluation of an order-p element's map and Jacobian, and a 3x3 solve."""
+    n1 = p + 1
+    return 12 * n1 ** 3 + 30 * n1 ** 2 + 18 * p * p + 80
 
 
 def _cpu_model() -> str:
@@ -162,8 +171,17 @@ def main() -> int:
     achieved_gbs = located_per_frame * bytes_per_sample / (k_ms * 1e-3) / 1e9
     walk = int(st.walk)   # the walk the library ran (the automatic choice depends on the frame's size)
     pol, shade = 'true' if args.polish else 'false', 2 if fp64_field else 0
-    # walk 5: the sample-parallel kernel (these frames have well over 32 rays per element column)
-    kernel_name = (f"k_integrate_binned<{p},{pol},{shade}>" if walk == 5 else f"k_integrate<{p},{pol},{walk},{shade}>")
+    kernel_name = (f"k_integrate_binned<{p},{pol},{shade}>" if st.binned else f"k_integrate_split<{p},{pol},{shade}>"
+                   if walk == 5 else f"k_integrate<{p},{pol},{walk},{shade}>")
+    if st.binned:
+        flops_per_sample = st.newton_steps / max(1, st.located_samples) * _newton_flops(p) + 2 * (p + 1) ** 3
+        achieved = located_per_frame * flops_per_sample / (k_ms * 1e-3) / 1e12
+        roofline = {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+                    "frac": achieved / FP32_PEAK_TFLOPS, "flops_per_unit": flops_per_sample}
+    else:
+        roofline = {"bound": "hbm", "achieved": achieved_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": achieved_gbs / HBM_PEAK_GBS, "bytes_per_unit": bytes_per_sample}
+    roofline.update(traffic=PMC_TRAFFIC_BYTES.get((args.config, kernel_name)), kernel=kernel_name, unit_name="located sample")
 
     out = {
         "metric": "located samples/s (volume render; also Mrays/s)",
@@ -193,10 +211,7 @@ def main() -> int:
         "integrate_kernel_ms": k_ms,
         "bvh_build_ms": {"cold": bvh_ms, "warm": bvh_ms_warm},
         "bvh_wide_nodes": int(bvh.wide_nodes.numel() // 64) if bvh.wide_nodes is not None else 0,
-        "roofline": {"bound": "hbm", "achieved": achieved_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved_gbs / HBM_PEAK_GBS, "traffic": PMC_TRAFFIC_BYTES.get((args.config, kernel_name)),
-                     "kernel": kernel_name,
-                     "bytes_per_unit": bytes_per_sample, "unit_name": "located sample"},
+        "roofline": roofline,
     }
 
     if args.error_sample:
