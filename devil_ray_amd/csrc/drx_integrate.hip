@@ -217,21 +217,29 @@ static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, con
   const double per_element = 64 * kBinnedR / (across * across * along);
   return per_column >= kBinnedMinRaysPerColumn && per_element >= (order == 4 ? kBinnedMinPointsOrder4 : kBinnedMinPoints);   // a NaN fails
 }
-// Do the rays of a block lie together?  Grouping pays where a wavefront finds its points' leaves by one descent and they
-// share elements: not for rays in no order or without the tile order, nor for small frames seen so obliquely that the box
-// around a wavefront's points is mostly empty.  Four wavefronts look at 64 consecutive rays of the processing order each, at
-// an eighth, three, five and seven eighths of it: the box around four consecutive samples of theirs half way along
-// the longest of the rays, in leaves (spread evenly over the bounds).  With three of the four boxes within the limit the
-// frame takes the grouping kernel (choice 1).  One block, in the place of the launch that clears the counters.  Up to
-// kChoiceWaitRays rays both forms are launched and one of them finds no rays (65,536 rays: 6 to 8 us); above, the host waits for
-// the choice (14 us) and launches one.
+// Do the rays of a block lie together, and do the leaves lie apart?  Grouping pays where a wavefront finds its points' leaves by
+// one descent, its points share elements and few of them have many candidates: not for rays in no order or without the
+// tile order, not for small frames seen so obliquely that the box around a wavefront's points is mostly empty, and not
+// for elements so sheared or elongated that their boxes overlap (a block goes round until its last point is settled).  Four
+// wavefronts look at 64 consecutive rays of the processing order each, at an eighth, three, five and seven eighths of
+// it: the box around four consecutive samples of theirs half way along the longest of the rays, and the leaves that
+// such a box overlaps on average inside the mesh, from 256 leaves spread over the tree: their boxes, and the room that their
+// elements fill.  With three of the four boxes within the limit,
+// and the leaves around a point within theirs, the frame takes the grouping kernel (choice 1).  One block, in the
+// place of the launch that clears the counters.  Up to kChoiceWaitRays rays both forms are launched and one of them finds no
+// rays (65,536 rays: 6 to 8 us); above, the host waits for the choice (14 us) and launches one.
 //
-// The limit by measurement, as above: time of the other form / of this one, least, median and most at leaves in the third
-// smallest box.  Against the per-lane sample-parallel form, order 1: 1.07, 1.31, 1.66 (up to 20), 1.09, 1.36, 1.46 (30-40), 0.78,
-// 1.00, 1.04 (60-70), 1.04, 1.09 (80-100), 0.76, 0.83, 0.86 (100-300); order 2: 1.19, 1.46, 1.81 (up to 20), 1.07, 1.11, 1.13
-// (60-70), 1.22, 1.28 (80-100), 0.79, 0.92, 1.03 (100-300); order 3: 1.39, 1.40 (80-100), 0.88, 1.07, 1.17 (150-300); order 4: 0.88,
-// 0.95, 1.04 (100-112), 1.02, 1.23, 1.53 (150-300), 0.86, 1.19, 1.38 (300-500); mixed 1-4: 1.11, 1.36, 1.65 (150-300).  Against
-// one lane per ray, orders 1-3: 0.91, 1.21, 1.33 (112-200).  Rays in no order have thousands.
+// The limits by measurement: time of the other form / of this one over 547 frames (orders 1-4, 3 to 60 elements an axis, warps up
+// to 0.18, 100^2 to 1000^2 rays, 40 to 600 samples, half of them oblique), least, median and most, against the per-lane
+// sample-parallel form, by leaves in the third smallest box and leaves around a point.  Order 1: 0.96, 1.20, 1.76 (0-40, up
+// to 1.5), 0.94, 1.29, 1.67 (0-40, 1.5-2.5), 0.73, 1.24, 1.49 (40-64, 1.5-2.5), 0.57, 0.78, 1.52 (40-64, 3.2-4), 0.77, 1.12, 1.36
+// (64-100, 1.5-2.5), 0.17, 0.41, 0.65 (40-100, above 4), 0.59, 0.67, 1.07 (100-300, 1.5-2.5).  Order 2: 0.99, 1.13, 1.58 (0-40,
+// up to 1.5), 0.76, 1.40, 1.75 (0-40, 4-5), 0.87, 1.14, 1.33 (40-64, 2.5-3.2), 1.01, 1.07, 1.44 (64-100, 1.5-2.5), 0.72, 0.74 (64-100,
+// 3.2-4), 0.64, 0.78, 1.07 (100-300, up to 2.5).  Order 3: 1.13, 1.59, 1.90 (0-40, 1.5-2.5), 1.09, 1.23, 1.42 (40-64, 2.5-3.2),
+// 0.99, 1.33, 1.45 (64-100, 1.5-2.5), 0.42 to 0.8 (64-100, above 3.2), 0.72, 0.88, 1.05 (100-300).  Order 4: 1.13, 1.28, 1.42
+// (64-100, 3.2-4), 0.91, 1.33, 1.40 (100-300, 1.5-2.5), 0.71, 0.82, 0.83 (100-300, 3.2-4).  Mixed 1-4: 1.11, 1.36, 1.65 (150-300,
+// about 1.3).  Against one lane per ray, orders 1-3: 0.91, 1.21, 1.33 (112-200, about 1.3), 0.38 to 0.68 (64-300, above 4).
+// Rays in no order have thousands of leaves in a box.
 //
 // And can rays end early?  A round locates 16 samples of a ray whether or not it is opaque after two.  Where a colour table's
 // largest opacity lets a ray end within kSamplesToEnd samples the other forms stay.  Time of the other form / of this one, least
@@ -240,29 +248,55 @@ static bool samples_share_elements (int order, int32_t n_rays, int32_t n_el, con
 // samples of a hundred, ends a ray after 25 at the earliest; up to 90 samples, where it may end one sooner, the forms are within
 // 12% of each other on eight domains of 4^3 to 10^3 elements.)
 constexpr int kSamplesToEnd = 24;
-constexpr float kBoxLeavesLowOrders = 100.f, kBoxLeaves = 300.f;
+constexpr float kBoxLeavesLowOrders = kBinLeaves, kBoxOverlapLowOrders = 180.f;   // leaves; leaves times leaves around a point
+constexpr float kBoxLeaves = 300.f, kBoxOverlap = 360.f;
 constexpr int32_t kChoiceWaitRays = 1 << 18;
 
-__global__ void __launch_bounds__ (256) k_integrate_choice (const Ray *__restrict__ rays, const int32_t *__restrict__ order, int n_rays,
-                                                            float sample_dist, float sx, float sy, float sz, float most_leaves,
-                                                            const float4 *__restrict__ lut, int lut_size, float opacity,
-                                                            int32_t *__restrict__ counters, int n_counters, int32_t *choice)
+struct ChoiceArgs
+{
+  const Ray *rays;
+  const int32_t *order;
+  int n_rays;
+  float sample_dist;
+  const float4 *leaf_boxes, *starts;   // starts: nullable, the leaves' Newton start maps
+  int n_leaves;
+  float volume;                // of the bounds
+  float most_leaves, most_overlap;
+  const float4 *lut;
+  int lut_size;
+  float opacity;
+  int32_t *counters, *choice;
+  int n_counters;
+};
+
+__global__ void __launch_bounds__ (256) k_integrate_choice (ChoiceArgs a)
 {
   __shared__ int32_t fit, opaque;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (threadIdx.x == 0) fit = opaque = 0;
-  if ((int)threadIdx.x < n_counters) counters[threadIdx.x] = 0;
+  if ((int)threadIdx.x < a.n_counters) a.counters[threadIdx.x] = 0;
   __syncthreads ();
-  const int64_t tile = ((int64_t)n_rays + 63) / 64 * (2 * wv + 1) / 8, i = 64 * tile + lane;
-  const bool has_ray = i < n_rays;
-  Ray ray = rays[has_ray ? (order ? order[i] : i) : 0];
+  const int64_t tile = ((int64_t)a.n_rays + 63) / 64 * (2 * wv + 1) / 8, i = 64 * tile + lane;
+  const bool has_ray = i < a.n_rays;
+  const Ray ray = a.rays[has_ray ? (a.order ? a.order[i] : i) : 0];
+  float4 b0[4], b1[4], m[4][3];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+  {
+    const int64_t leaf = (int64_t)(64 * q + lane) * a.n_leaves / 256;
+    b0[q] = a.leaf_boxes[2 * leaf];
+    b1[q] = a.leaf_boxes[2 * leaf + 1];
+    if (a.starts)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) m[q][d] = a.starts[3 * leaf + d];
+  }
   const float half = 0.5f * wave_reduce_max (has_ray ? ray.far_ - ray.near_ : 0.f);
   float lo[3] = { INFINITY, INFINITY, INFINITY }, hi[3] = { -INFINITY, -INFINITY, -INFINITY };
 #pragma unroll
   for (int q = 0; q < 4; ++q)
   {
-    const float t = ray.near_ + half + q * sample_dist;
-    if (has_ray && t - sample_dist < ray.far_)
+    const float t = ray.near_ + half + q * a.sample_dist;
+    if (has_ray && t - a.sample_dist < ray.far_)
 #pragma unroll
       for (int d = 0; d < 3; ++d)
       {
@@ -271,16 +305,33 @@ __global__ void __launch_bounds__ (256) k_integrate_choice (const Ray *__restric
         hi[d] = fmaxf (hi[d], x);
       }
   }
-  const float scale[3] = { sx, sy, sz };
-  float leaves = 1.f;
+  float box[3];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) leaves *= 1.f + fmaxf (wave_reduce_max (hi[d]) - wave_reduce_min (lo[d]), 0.f) * scale[d];
-  if (lane == 0 && leaves <= most_leaves) atomicAdd (&fit, 1);
+  for (int d = 0; d < 3; ++d) box[d] = fmaxf (wave_reduce_max (hi[d]) - wave_reduce_min (lo[d]), 0.f);
+  float in_box = 0.f, at_point = 0.f, filled = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+  {
+    const float l0 = b0[q].w - b0[q].x, l1 = b1[q].x - b0[q].y, l2 = b1[q].y - b0[q].z;
+    in_box += (box[0] + l0) * (box[1] + l1) * (box[2] + l2);
+    at_point += l0 * l1 * l2;
+    if (a.starts)   // the leaf's share of its element: the start map takes the element to the unit cube
+    {
+      const float det = m[q][0].x * (m[q][1].y * m[q][2].z - m[q][1].z * m[q][2].y) -
+                        m[q][0].y * (m[q][1].x * m[q][2].z - m[q][1].z * m[q][2].x) +
+                        m[q][0].z * (m[q][1].x * m[q][2].y - m[q][1].y * m[q][2].x);
+      filled += fminf (1.f / (DRX_SPLITS_PER_ELEMENT * fabsf (det)), l0 * l1 * l2);
+    }
+  }
+  filled = a.starts ? wave_reduce_add (filled) : 256.f * a.volume / a.n_leaves;
+  in_box = wave_reduce_add (in_box) / filled;
+  at_point = wave_reduce_add (at_point) / filled;
+  if (lane == 0 && in_box <= a.most_leaves && in_box * at_point <= a.most_overlap) atomicAdd (&fit, 1);   // a NaN fails
   bool ends = false;
-  for (int q = threadIdx.x; q < lut_size; q += 256) ends = ends || !(lut[q].w < opacity);   // a NaN is none to rely on
+  for (int q = threadIdx.x; q < a.lut_size; q += 256) ends = ends || !(a.lut[q].w < a.opacity);   // a NaN is none to rely on
   if (ends) atomicOr (&opaque, 1);
   __syncthreads ();
-  if (threadIdx.x == 0) *choice = fit >= 3 && !opaque ? 1 : 0;
+  if (threadIdx.x == 0) *a.choice = fit >= 3 && !opaque ? 1 : 0;
 }
 
 constexpr int kIntWaves = kIntBlock / 64;
@@ -1025,6 +1076,10 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   // Sample-parallel launch: asked for, or picked for frames of fewer than kSplitMaxRaysPerSimd active rays per SIMD
   // under the automatic walk and launch.  In its place, and in the place of one lane per ray, frames whose samples share
   // elements take k_integrate_binned, but for small BVHs that carry the 8-wide copy (the wave walk) in large frames.
+  // There the line stands where the wave walk's rule had drawn it, not where the times say; wave walk / k_integrate_binned,
+  // ms: 12^3 order 1, 700^2 rays 0.28 / 0.35 (8 samples across the bounds), 0.57 / 0.47 (24), 1.39 / 0.74 (64), 4.27 / 1.85
+  // (200); 12^3 order 2, 1100^2, oblique 0.57 / 0.84, 1.03 / 1.20, 2.30 / 2.06, 6.88 / 5.38; 6^3 order 3, 700^2 0.37 / 0.38,
+  // 0.96 / 0.61, 2.42 / 1.20, 7.55 / 3.08; 12^3 order 4, 1100^2 0.45 / 0.59, 1.11 / 0.89, 2.85 / 1.92, 9.14 / 4.99.
   const int launch = opts ? opts->launch : DRX_LAUNCH_AUTO;
   const bool plain = !guided && !learned && P <= DRX_MAX_MIXED_ORDER;
   bool split = false, binned = false;
@@ -1041,7 +1096,7 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
     split = hipGetDevice (&dev) == hipSuccess && (int64_t)n_rays < (int64_t)kSplitMaxRaysPerSimd * 4 * compute_units (dev);
     binned = split || !(a.cfg.wide && bvh->n_leaves <= kWaveWalkMaxLeaves);
   }
-  binned = binned && samples_share_elements (P, n_rays, mesh->n_el, bvh->bounds, sample_dist);
+  binned = binned && a.cfg.qnodes && samples_share_elements (P, n_rays, mesh->n_el, bvh->bounds, sample_dist);
   int walk = split ? DRX_TRAVERSE_BINARY : trav;
   if (walk == DRX_TRAVERSE_AUTO && a.cfg.wide && !learned && P <= DRX_MAX_MIXED_ORDER)
   {
@@ -1208,16 +1263,13 @@ int drx_volume_integrate (const drx_mesh *mesh, const drx_mesh *field, const drx
   const int n_counters = 16;
   if (binned)
   {
-    float scale[3];
-    const float per_axis = std::cbrt ((float)bvh->n_leaves);
-    for (int d = 0; d < 3; ++d)
-    {
-      const float ext = bvh->bounds[2 * d + 1] - bvh->bounds[2 * d];
-      scale[d] = ext > 0.f ? per_axis / ext : 0.f;
-    }
-    const float most = split && (P == 1 || P == 2) ? kBoxLeavesLowOrders : kBoxLeaves;
-    hipLaunchKernelGGL (k_integrate_choice, dim3 (1), dim3 (256), 0, st, a.rays, a.order, n_rays, sample_dist, scale[0], scale[1],
-                        scale[2], most, a.lut, lut_size, 1.f - std::pow (0.05f, 1.f / kSamplesToEnd), (int32_t *)dstats, n_counters, err + 2);
+    const bool low = split && P >= 1 && P <= 3;
+    const float *e = bvh->bounds;
+    const ChoiceArgs c { a.rays, a.order, n_rays, sample_dist, a.cfg.leaf_boxes, (const float4 *)bvh->leaf_starts, bvh->n_leaves,
+                         (e[1] - e[0]) * (e[3] - e[2]) * (e[5] - e[4]), low ? kBoxLeavesLowOrders : kBoxLeaves,
+                         low ? kBoxOverlapLowOrders : kBoxOverlap, a.lut, lut_size,
+                         1.f - std::pow (0.05f, 1.f / kSamplesToEnd), (int32_t *)dstats, err + 2, n_counters };
+    hipLaunchKernelGGL (k_integrate_choice, dim3 (1), dim3 (256), 0, st, c);
   }
   else
     hipLaunchKernelGGL (k_fill_i32q, dim3 (1), dim3 (64), 0, st, (int32_t *)dstats, (int64_t)n_counters, 0);

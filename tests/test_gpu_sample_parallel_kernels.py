@@ -40,7 +40,7 @@ FINE = [
     ("p1_n16", lambda: syn.hex_mesh(16, 1, 0.05, 0.01, 3), (0.5, 0.5, 3.0), 240, 300, False, False, False),
     ("p2_n14_fp64_field", lambda: syn.hex_mesh(14, 2, 0.05, 0.01, 5, keep_field64=True), (2.2, 2.0, 2.3), 330, 300, False, False,
      True),
-    ("p3_n12_lit", lambda: syn.hex_mesh(12, 3, 0.15, 0.01, 4), (-1.4, 1.9, 2.0), 230, 170, True, False, False),
+    ("p3_n12_lit", lambda: syn.hex_mesh(12, 3, 0.1, 0.01, 4), (-1.4, 1.9, 2.0), 300, 220, True, False, False),
     ("p4_n10_polish", lambda: syn.hex_mesh(10, 4, 0.2, 0.01, 6), (2.2, 2.0, 2.3), 200, 130, False, True, False),
     ("mixed_n10", lambda: syn.mixed_hex_mesh(10, 0.1, 0.01, 7), (2.2, 2.0, 2.3), 210, 150, False, False, False),
     ("p3_n12_inside", lambda: syn.hex_mesh(12, 3, 0.1, 0.01, 8), (0.52, 0.48, 0.55), 120, 160, False, True, False),
@@ -104,7 +104,7 @@ def test_coarse_march_per_lane(gpu, p):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,p,side", [(12, 3, 300), (14, 2, 640)])
+@pytest.mark.parametrize("n,p,side", [(12, 3, 304), (14, 2, 640)])   # whole tiles
 def test_rays_in_no_order_per_lane(gpu, n, p, side):
     """The form is chosen by how the rays lie in processing order: grouped in tile order; a sample (small frame) or a ray
     (more than 300 active rays per SIMD) per lane for the same rays shuffled.  The partials of a ray are the same."""
@@ -168,3 +168,15 @@ def test_many_candidates_counted(gpu):
     rays["orig"][:, 0], rays["orig"][:, 1], rays["orig"][:, 2] = np.tile(g, side), -0.5, np.repeat(g, side)
     rays["dir"] = (1e-7, 1.0, 1e-7)
     _compare(gpu, mesh, gpu.as_bytes(rays), side, 160, False, False, False, 0, alpha=0.2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p,shear", [(2, 0.0), (2, 8.0), (3, 5.0)])
+def test_sheared_elements_per_lane(gpu, p, shear):
+    """Elements sheared over several of their widths: their boxes overlap, some points have many candidates, and the form
+    that goes round until all are settled is not taken."""
+    mesh = syn.hex_mesh(8, p, 0.02, 0.01, 3)
+    mesh.values[:, 0] += np.float32(shear) * mesh.values[:, 2]
+    c = 0.5 * (1.0 + shear)
+    cam = gpu.Camera(200, 200, 45.0, pos=(c, 0.5, 2.5 + shear), look_at=(c, 0.5, 0.5))
+    _compare(gpu, mesh, cam.create_rays(), 200, 300, False, False, False, 0 if shear else 1)
