@@ -1010,10 +1010,10 @@ int drx_bvh_quantize (const drx_bvh *bvh, uint32_t *out_qnodes, float *out_leaf_
   return DRX_OK;
 }
 
-// One cell per 16 to 32 leaves, as near to cubes as powers of two allow, 2^24 at most.  Measured on the 64^3 order-3
-// mesh (2^24 > leaves > 2^23), 1024^2 frame, integrate kernel without cells 13.85 ms; cells / cost of making them:
-// 2^19 13.12 ms / 98 us, 2^20 12.66 ms / 163 us, 2^21 12.63 ms / 292 us, 2^23 13.09 ms / 1.05 ms (finer cells miss
-// the caches); 40^3 order 4: 84.1 -> 73.2 ms with 2^18.
+// One cell per 8 to 16 leaves (more where an axis has 2^12 cells already), as near to cubes as powers of two allow, 2^24 at
+// most.  Measured on the 64^3 order-3 mesh (2^24 > leaves > 2^23: 2^20 cells), 1024^2 frame, integrate kernel without cells
+// 13.85 ms; cells / cost of making them: 2^19 13.12 ms / 98 us, 2^20 12.66 ms / 163 us, 2^21 12.63 ms / 292 us, 2^23 13.09 ms
+// / 1.05 ms (finer cells miss the caches); 40^3 order 4: 84.1 -> 73.2 ms with 2^18.
 constexpr int kEntryLog2LeavesPerCell = 4;
 
 int64_t drx_bvh_entry_bits (int32_t n_leaves, const float *bounds6, int32_t *out_bits)

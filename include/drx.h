@@ -221,8 +221,9 @@ typedef struct drx_integrate_stats
                                  element, 0 the one that locates a sample per lane; 0 for every other walk.  The
                                  first runs where neighbouring samples share elements: at least 32 active rays per
                                  element column, steps and pixels short against an element, 64 consecutive rays of
-                                 the processing order lying together, no ray opaque within 24 samples, no sample
-                                 with 128 candidates */
+                                 the processing order lying together, leaf boxes that overlap little, no ray opaque
+                                 within 24 samples, no sample that 128 candidates leave unlocated; and the BVH
+                                 carries compact nodes */
 } drx_integrate_stats;
 
 /* PointLight (rendering/point_light.hpp:15-33); dray's defaults: amb 0.4, diff 0.75, spec 0.8, spec_pow 15. */
