@@ -228,7 +228,16 @@ __global__ void __launch_bounds__ (256) k_entry_cells (const uint4 *__restrict__
 // 1.97 ms chunked by 256 and 1.94 / 2.30 ms by 64; 1 M: 0.77 / 0.72 ms against 0.72 / 0.76 ms by 64; learned, 8 M
 // plain: 5.80 ms against 6.79 ms by 64).  Unordered points of the plain walk gain nothing from refill, and at that
 // size 1,024 is as good as 64 (4 M, order 3: 3.56 ms against 3.65 ms).
-constexpr int kLocateChunk = 64, kLocateChunkRefill = 128, kLocateChunkLarge = 1024, kLocateRefillRounds = 4;
+// The queue hands out about 75 chunks a microsecond, so a persistent launch by 128 takes at least 0.1 ms per million points,
+// whatever they cost.  Elements of order 1 cost less, those of order 2 not much more, and points outside the mesh nothing:
+// chunks of 256 without a queue there, chunks of 256 from the queue for many points (persistent by 128 / chunked by 256 /
+// persistent by 256, ms, means of two meshes of 14^3 to 50^3 elements: order 1: 4 M in a box 0.005 wide 0.48 / 0.21 / - (30^3),
+// 12 M in a plane 1.22 / 0.75 / - (30^3), a grid of 16 M 1.85 / 1.70 / 1.80; order 2: 4 M random 0.97 / 0.97 / 0.98, 16 M
+// 3.15 / 3.28 / 3.14, 16 M along rays 2.43 / 2.59 / 2.41, mostly outside 1.57 / 0.88 / 1.06; order 3: 16 M random 3.72 / 3.96 / 3.69,
+// mostly outside 1.63 / 1.15 / 1.28; order 4: 16 M random 4.24 / 4.59 / 4.20, along rays 3.67 / 4.21 / 3.64, mostly outside
+// 1.72 / 1.23 / 1.35; mixed and learned, 16 M: by 256 from the queue 1.00 to 1.04x, mostly outside 1.17 to 1.23x).
+constexpr int kLocateChunk = 64, kLocateChunkRefill = 128, kLocateChunkMany = 256, kLocateChunkLarge = 1024, kLocateRefillRounds = 4;
+constexpr int64_t kLocateManyPoints = 6 << 20;
 
 // Does the order of many points pay for its sort?  Points in no spatial order make every lane of a wavefront read nodes
 // and element nets of its own; sorted, lanes share them.  Sort + walk against walk alone, random points, order 1 / 2 /
@@ -1136,8 +1145,12 @@ static int locate_impl (const drx_mesh *mesh, const drx_bvh *bvh, const float *p
   const int64_t resident = (int64_t)compute_units (dev) * 4 * locate_waves_per_simd (P, cfg.polish, learned ? 3 : walk);
   // (a chunk of 64 is for small n only, so the grid's work-item count, 64 per chunk, stays in 32 bits)
   const bool large = n > 64 * kLocateRefillRounds * resident, ordered = learned || by_size || sort;
-  if (launch == DRX_LAUNCH_AUTO) launch = large && ordered && chunk == 0 ? DRX_LAUNCH_PERSISTENT : DRX_LAUNCH_CHUNKED;
-  if (chunk == 0) chunk = !large ? kLocateChunk : launch == DRX_LAUNCH_PERSISTENT ? kLocateChunkRefill : kLocateChunkLarge;
+  const bool many = n >= kLocateManyPoints, queued = learned || P == 0 || P >= 3 || (P == 2 && many);
+  if (launch == DRX_LAUNCH_AUTO) launch = large && ordered && queued && chunk == 0 ? DRX_LAUNCH_PERSISTENT : DRX_LAUNCH_CHUNKED;
+  if (chunk == 0)
+    chunk = !large ? kLocateChunk
+            : launch == DRX_LAUNCH_PERSISTENT ? (many ? kLocateChunkMany : kLocateChunkRefill)
+            : ordered ? kLocateChunkMany : kLocateChunkLarge;
   if (chunk < 64 || chunk > (1 << 20)) return fail (DRX_ERR_ARG, "drx_locate: chunk %d outside [64, 2^20]", chunk);
   const int64_t n_chunks = (n + chunk - 1) / chunk;
   if (n_chunks > (1ll << 31) - 1) return fail (DRX_ERR_ARG, "drx_locate: too many chunks");

@@ -6,6 +6,7 @@
 int fake_fail_malloc = -1, fake_fail_launch = -1;   /* index of the call that fails */
 int fake_mallocs = 0, fake_launches = 0, fake_copies = 0, fake_first_copy = 0;
 long fake_live = 0;                                 /* bytes of device memory held */
+unsigned fake_grid = 0;                             /* blocks of the last launch */
 static int last_error = 0;
 
 static int failed (int e) { return last_error = e; }
@@ -43,7 +44,12 @@ int hipMemcpyAsync (void *d, const void *s, size_t n, int k, void *st)
   return 0;
 }
 typedef struct { unsigned x, y, z; } dim3;
-int __hipPushCallConfiguration (dim3 g, dim3 b, size_t s, void *st) { (void)g; (void)b; (void)s; (void)st; return 0; }
+int __hipPushCallConfiguration (dim3 g, dim3 b, size_t s, void *st)
+{
+  (void)b; (void)s; (void)st;
+  fake_grid = g.x;
+  return 0;
+}
 int __hipPopCallConfiguration (dim3 *g, dim3 *b, size_t *s, void **st)
 {
   g->x = g->y = g->z = b->x = b->y = b->z = 1;

@@ -1,6 +1,6 @@
 """When drx_locate sorts by itself, and what it does where the sort's memory or a launch fails (on the CPU, over
 tests/fake_hip.c): without room for the sort the points are taken as they come, nothing is kept and no error is left; a
-failing launch is reported."""
+failing launch is reported.  And how it launches the points that it finds in order."""
 import json
 import os
 import subprocess
@@ -19,14 +19,15 @@ from devil_ray_amd import _lib as L
 lib = L.lib()
 get = lambda n, t=C.c_int: t.in_dll(fake, n)
 get("fake_fail_malloc").value, get("fake_fail_launch").value = int(sys.argv[3]), int(sys.argv[4])
-get("fake_first_copy").value = 1 << 20
+get("fake_first_copy").value = int(sys.argv[9])
 n = int(sys.argv[5])
 buf = C.create_string_buffer(64)
 at = C.addressof(buf)
 m, b, o = L.DrxMesh(), L.DrxBVH(), L.DrxLocateOpts()
-m.data, m.n_el, m.order, m.ncomp, m.stride = at, 1000, 3, 3, lib.drx_mesh_stride(3, 3)
+order = int(sys.argv[8])
+m.data, m.n_el, m.order, m.ncomp, m.stride = at, 1000, order, 3, lib.drx_mesh_stride(order, 3)
 b.inner_nodes = b.leaf_pack = b.leaf_nodes = b.aabb_ids = b.subrefs = at
-b.n_leaves = 33000
+b.n_leaves = 33000 if order > 1 else 66000
 b.bounds[:] = [0, 1, 0, 1, 0, 1]
 o.coherent_order = int(sys.argv[6])
 if int(sys.argv[7]):   # mixed orders
@@ -34,7 +35,7 @@ if int(sys.argv[7]):   # mixed orders
     m.order, m.stride = int(sys.argv[7]), 0
 rc = lib.drx_locate(C.byref(m), C.byref(b), at, n, at, C.byref(o), None)
 print(json.dumps([rc, (lib.drx_last_error() or b"").decode(), get("fake_mallocs").value, get("fake_launches").value,
-                  get("fake_live", C.c_long).value]))
+                  get("fake_live", C.c_long).value, get("fake_grid").value]))
 """
 
 
@@ -45,11 +46,12 @@ def fake(tmp_path_factory):
     return so
 
 
-def _run(fake, fail_malloc=-1, fail_launch=-1, n=N, coherent=0, mixed=0):
+def _run(fake, fail_malloc=-1, fail_launch=-1, n=N, coherent=0, mixed=0, order=3, far=1 << 20, grid=False):
     r = subprocess.run([sys.executable, "-c", CHILD, fake, os.path.dirname(HERE), str(fail_malloc), str(fail_launch), str(n),
-                        str(coherent), str(mixed)], capture_output=True, text=True, timeout=120)
+                        str(coherent), str(mixed), str(order), str(far)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-2000:]
-    return json.loads(r.stdout.strip().splitlines()[-1])
+    out = json.loads(r.stdout.strip().splitlines()[-1])
+    return out if grid else out[:5]
 
 
 def test_no_room_for_the_sort(fake):
@@ -76,3 +78,14 @@ def test_mixed_orders_sort_from(fake, order, least):
     """A mesh of mixed orders whose largest is 4 is not taken for one of order 4: most of its elements may be of order 1."""
     assert _run(fake, n=least - 1, mixed=order)[2] == 1   # the flags alone
     assert _run(fake, n=least, mixed=order)[2] == 7
+
+
+@pytest.mark.parametrize("order,n,chunked", [(1, 4 << 20, True), (1, 16 << 20, True), (2, 4 << 20, True), (2, 8 << 20, False),
+                                             (3, 4 << 20, False), (4, 16 << 20, False)])
+@pytest.mark.parametrize("far", [0, 1 << 20])
+def test_cheap_elements_take_no_queue(fake, order, n, chunked, far):
+    """The persistent launch's queue bounds points that cost little: order 1, and order 2 below 6 M points, go by chunks of
+    256 whether they were found in order (far 0) or sorted."""
+    rc, text, mallocs, _, _, grid = _run(fake, n=n, order=order, far=far, grid=True)
+    assert (rc, text) == (0, "") and mallocs == (7 if far else 1)
+    assert grid == n // 256 if chunked else grid < n // 256   # chunked: a wavefront for each; else the resident ones
