@@ -88,7 +88,7 @@ __device__ __forceinline__ float clamp01f (float v) { return fminf (1.f, fmaxf (
 // ambient + diffuse + Blinn-Phong specular, gradient flipped toward the light and the half vector
 // (flips persist across lights), channels clamped after each light; alpha <= 0.01 gives zero.
 template <int P, typename G>
-__device__ __forceinline__ float4 lit_color_at (const IntegrateArgs &a, G g, G f, const float ref[3], const float dir[3])
+__device__ float4 lit_color_at (const IntegrateArgs &a, G g, G f, const float ref[3], const float dir[3])
 {
   float y[3], J[3][3];
   eval_geom<P, float> (g, ref, y, J);
@@ -336,9 +336,17 @@ __global__ void __launch_bounds__ (256) k_integrate_choice (ChoiceArgs a)
 
 constexpr int kIntWaves = kIntBlock / 64;
 
+// The lit binary walks of order 2 with the FP64 correction spill 100 registers at five waves per SIMD, and since they start
+// from entry cells too many of them in the inner loops: 24^3 elements, 600^2 orthographic rays x 194 samples 9.0 ms before the
+// cells, 11.0 ms with them; at four waves 7.4 ms.
+__host__ __device__ constexpr int integrate_waves_per_simd (int P, bool polish, int mode, int shade)
+{
+  return P == 2 && polish && shade == 1 && (mode == 0 || mode == 4) ? 4 : waves_per_simd (P, polish, mode);
+}
+
 // SHADE: 0 VolumeShader::color over an FP32 field, 1 shaded_color (lit), 2 color over an FP64 field.
 template <int P, bool POLISH, int MODE, int SHADE>
-__global__ void __launch_bounds__ (kIntBlock, waves_per_simd (P, POLISH, MODE)) k_integrate (IntegrateArgs a)
+__global__ void __launch_bounds__ (kIntBlock, integrate_waves_per_simd (P, POLISH, MODE, SHADE)) k_integrate (IntegrateArgs a)
 {
   constexpr bool LIT = SHADE == 1;
   constexpr bool WAVE = MODE == 2;
