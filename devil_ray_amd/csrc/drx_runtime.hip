@@ -264,9 +264,12 @@ __global__ void __launch_bounds__ (kScanBlock) k_scan_down (const int32_t *in, i
   }
 }
 
-// Small arrays (the digit counts of a sort of up to half a million keys, the flags of small frames): one block walks the
-// array with a carry, one launch instead of three (8,704 counts: 10 us against 12 us and two launches).
-constexpr int kScanSmallBlock = 1024, kScanSmallItems = 8, kScanSmallMax = 4 * kScanSmallBlock * kScanSmallItems;
+// Small arrays (the digit counts of a sort of up to 160 K keys, the flags of small frames): one block walks the array with a
+// carry, one launch instead of three (8,704 counts: 10 us against 12 us and two launches).  Each further 8 K counts cost the
+// block 4 us, three launches next to nothing: domains' partials composited (7 scans each), ms by one block / by three launches:
+// 140 K partials (8,960 counts) 0.221 / 0.229, 160 K (10,240) 0.225 / 0.227, 200 K (12,544) 0.245 / 0.234, 300 K 0.282 / 0.245,
+// 500 K (31,488) 0.376 / 0.260; a BVH of 456 K leaves (4 scans) 0.444 / 0.387.
+constexpr int kScanSmallBlock = 1024, kScanSmallItems = 8, kScanSmallMax = 10 << 10;
 
 __global__ void __launch_bounds__ (kScanSmallBlock) k_scan_small (const int32_t *in, int32_t *out, int32_t n, int32_t *sum,
                                                                    int32_t *total)

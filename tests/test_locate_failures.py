@@ -89,3 +89,9 @@ def test_cheap_elements_take_no_queue(fake, order, n, chunked, far):
     rc, text, mallocs, _, _, grid = _run(fake, n=n, order=order, far=far, grid=True)
     assert (rc, text) == (0, "") and mallocs == (7 if far else 1)
     assert grid == n // 256 if chunked else grid < n // 256   # chunked: a wavefront for each; else the resident ones
+
+
+def test_scans_of_a_sort(fake):
+    """A radix pass counts the digits of 4,096 keys at a time; up to 10,240 counts are scanned by one launch, more by three."""
+    one, last, three = (_run(fake, n=n, coherent=1)[3] for n in (8192, 40 * 4096, 40 * 4096 + 1))
+    assert one == last and three == last + 2 * 3   # three passes
